@@ -174,4 +174,10 @@ int hk_attention_reference(struct h3_gpu *gpu, const uint16_t *q,
                            uint32_t q_rows, uint32_t kv_rows, uint32_t heads,
                            uint32_t head_dim, float scale, int head_major);
 
+/* C[M,N] = X[M,K] . W[N,K]^T (+ bias) in F32 on the matrix cores; false (and
+ * nothing launched) for a shape or alignment it does not take. */
+bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
+                   const float *bias, float *c, uint32_t m, uint32_t n,
+                   uint32_t k);
+
 #endif

@@ -2214,7 +2214,10 @@ int h3_gpu_linear_f32(h3_gpu *gpu, h3_gpu_tensor *output,
         !hk_require_active(gpu))
         return 0;
     hk_op_begin(gpu, "linear_f32");
-    if (rows && output_dim)
+    if (rows && output_dim &&
+        !hk_linear_f32(gpu, HK_CF32(input), HK_CF32(weight),
+                       bias ? HK_CF32(bias) : (const float *)NULL,
+                       HK_F32(output), rows, output_dim, input_dim))
         hipLaunchKernelGGL(hk_linear_f32_kernel,
                            dim3((output_dim + 255) / 256, rows), dim3(256), 0,
                            gpu->stream, HK_CF32(input), HK_CF32(weight),
