@@ -180,4 +180,11 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
                    const float *bias, float *c, uint32_t m, uint32_t n,
                    uint32_t k);
 
+/* The F32 patch projection into bf16 rows (row r to row_map[r], or to r with
+ * a null map), in the sequential kernel's own fmaf order; false as above. */
+bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
+                     const float *bias, uint16_t *out,
+                     const uint32_t *row_map, uint32_t m, uint32_t n,
+                     uint32_t k);
+
 #endif

@@ -1,5 +1,5 @@
 /* Small projections of the DiT path on the matrix cores: the F32 linears of
- * the timestep MLP.
+ * the timestep MLP and the F32 patch projections.
  *
  * F32 MFMAs (v_mfma_f32_16x16x4_f32) multiply and add in full F32: measured
  * on the card, each of their k steps is one fmaf of the accumulator, in k
@@ -142,5 +142,135 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
         hk_linear_f32_run<3, 4>(gpu, x, w, bias, c, m, n, k);
     else
         hk_linear_f32_run<4, 4>(gpu, x, w, bias, c, m, n, k);
+    return true;
+}
+
+/* ------------------------------------------------------ patch projection
+ *
+ * F32 in, bf16 out, and bit for bit the reference's hand kernel
+ * (h3_cuda_core.cu:374-403): fmaf from the bias in k order.  The F32 MFMA
+ * keeps that order (above), so each accumulator starts at the bias and runs
+ * through k four at a time, lane quarter q holding k = 4 s + q.
+ *
+ * Bound by the F32 MFMA rate (1.85 GFLOP for 1792 x 96 -> 5376, 12 us at
+ * 157 TFLOP/s; its bytes take 4 us).  A 128-column x 64-row tile per
+ * workgroup (four waves of 64 x 32) gives the checkpoint's 5376 columns
+ * 42 x 28 workgroups at 1792 rows and 27 KiB of LDS lets four share a CU, so
+ * one's loads overlap the others' MFMAs.  LDS holds each row's 32-deep k
+ * chunk quarter by quarter (k % 4, then k / 4), so that one 16-byte read
+ * feeds four MFMAs; a row pitch of 36 floats spreads 16 rows over all banks.
+ * One thread per output had read W rows with a 384-byte stride between
+ * lanes: 31.5 us from 493 at 1792 rows, 4.8 from 9.6 at 74 (32 inputs). */
+enum { HK_PL_COLS = 128, HK_PL_ROWS = 64, HK_PL_K = 32, HK_PL_PITCH = 36 };
+
+__global__ void __launch_bounds__(256)
+hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
+                     uint16_t *out, const uint32_t *row_map, uint32_t m,
+                     uint32_t n, uint32_t k) {
+    __shared__ __attribute__((aligned(16)))
+    float lds[(HK_PL_COLS + HK_PL_ROWS) * HK_PL_PITCH];
+    float *lds_x = lds + HK_PL_COLS * HK_PL_PITCH;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t r16 = lane & 15u, quad = lane >> 4;
+    const uint32_t n0 = blockIdx.x * HK_PL_COLS, m0 = blockIdx.y * HK_PL_ROWS;
+    const uint32_t wn = (wave >> 1) * 64u, wm = (wave & 1u) * 32u;
+    /* staging: thread t takes 16-byte piece t % 8 of rows t / 8 + 32 i;
+     * rows past the end repeat the last one (their outputs are dropped) */
+    const uint32_t piece = tid & 7u, srow = tid >> 3;
+    const float *wp[4], *xp[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++)
+        wp[i] = w + (size_t)min(n0 + srow + 32u * i, n - 1u) * k + piece * 4u;
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++)
+        xp[i] = x + (size_t)min(m0 + srow + 32u * i, m - 1u) * k + piece * 4u;
+    hk_f32x4 wv[4], xv[2];
+    auto load = [&](uint32_t k0) {
+        if (k0 + piece * 4u >= k) return;
+#pragma unroll
+        for (int i = 0; i < 4; i++) wv[i] = *(const hk_f32x4 *)(wp[i] + k0);
+#pragma unroll
+        for (int i = 0; i < 2; i++) xv[i] = *(const hk_f32x4 *)(xp[i] + k0);
+    };
+    auto put = [&](float *base, hk_f32x4 v) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) base[e * 8 + piece] = v[e];
+    };
+    hk_f32x4 acc[4][2];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t col = n0 + wn + 16u * a + quad * 4u + i;
+            const float b = bias && col < n ? bias[col] : 0.0f;
+            acc[a][0][i] = acc[a][1][i] = b;
+        }
+#pragma unroll
+    for (int i = 0; i < 4; i++) wv[i] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    xv[0] = xv[1] = wv[0];
+    load(0);
+    for (uint32_t k0 = 0; k0 < k; k0 += HK_PL_K) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++)
+            put(lds + (srow + 32u * i) * HK_PL_PITCH, wv[i]);
+#pragma unroll
+        for (uint32_t i = 0; i < 2; i++)
+            put(lds_x + (srow + 32u * i) * HK_PL_PITCH, xv[i]);
+        __syncthreads();
+        if (k0 + HK_PL_K < k) load(k0 + HK_PL_K);
+        const uint32_t steps = min((k - k0) / 4u, 8u);
+#pragma unroll
+        for (uint32_t g = 0; g < 2; g++) {
+            hk_f32x4 wf[4], xf[2];
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+                wf[a] = *(const hk_f32x4 *)(
+                    lds + (wn + 16u * a + r16) * HK_PL_PITCH + quad * 8u +
+                    g * 4u);
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+                xf[b] = *(const hk_f32x4 *)(
+                    lds_x + (wm + 16u * b + r16) * HK_PL_PITCH + quad * 8u +
+                    g * 4u);
+#pragma unroll
+            for (uint32_t s = 0; s < 4; s++)
+                if (g * 4u + s < steps)
+#pragma unroll
+                    for (int a = 0; a < 4; a++)
+#pragma unroll
+                        for (int b = 0; b < 2; b++)
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                wf[a][s], xf[b][s], acc[a][b], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const uint32_t row = m0 + wm + 16u * b + r16;
+        if (row >= m) continue;
+        uint16_t *dst = out + (size_t)(row_map ? row_map[row] : row) * n;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const uint32_t col = n0 + wn + 16u * a + quad * 4u;
+            if (col < n)
+                *(uint2 *)(dst + col) =
+                    make_uint2(hk_pack2(acc[a][b][0], acc[a][b][1]),
+                               hk_pack2(acc[a][b][2], acc[a][b][3]));
+        }
+    }
+}
+
+bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
+                     const float *bias, uint16_t *out,
+                     const uint32_t *row_map, uint32_t m, uint32_t n,
+                     uint32_t k) {
+    if (!k || k % 4 || n % 4 || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
+        ((uintptr_t)out & 7) || m > 65535u * HK_PL_ROWS)
+        return false;
+    hipLaunchKernelGGL(hk_patch_linear_mfma,
+                       dim3((n + HK_PL_COLS - 1) / HK_PL_COLS,
+                            (m + HK_PL_ROWS - 1) / HK_PL_ROWS),
+                       dim3(256), 0, gpu->stream, x, w, bias, out, row_map, m,
+                       n, k);
     return true;
 }

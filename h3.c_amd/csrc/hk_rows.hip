@@ -2057,13 +2057,16 @@ static int hk_patch_common(h3_gpu *gpu, uint16_t *out,
                            uint32_t input_dim, uint32_t output_dim,
                            const char *name) {
     hk_op_begin(gpu, name);
-    if (rows && output_dim)
+    const float *x = HK_CF32(input) + input_offset;
+    const float *b = bias ? HK_CF32(bias) : (const float *)NULL;
+    if (rows && output_dim &&
+        !hk_patch_linear(gpu, x, HK_CF32(weight), b, out, row_map, rows,
+                         output_dim, input_dim))
         hipLaunchKernelGGL(hk_patch_linear_kernel,
                            dim3((output_dim + 255) / 256, rows), dim3(256),
-                           input_dim * sizeof(float), gpu->stream,
-                           HK_CF32(input) + input_offset, HK_CF32(weight),
-                           bias ? HK_CF32(bias) : (const float *)NULL, out,
-                           row_map, rows, input_dim, output_dim);
+                           input_dim * sizeof(float), gpu->stream, x,
+                           HK_CF32(weight), b, out, row_map, rows, input_dim,
+                           output_dim);
     return hk_op_end(gpu, name, HK_KIND_DIRECT);
 }
 

@@ -182,6 +182,8 @@ def lib():
                                                  _U32, _U32, _U32]),
         "h3_gpu_patch_linear_bf16_map": (_I, [_P, _P, _P, _P, _P, _P, _U32,
                                               _U32, _U32, _U32]),
+        "h3_hip_patch_linear_bf16_map": (_I, [_P, _P, _P, _P, _P, _P, _U32,
+                                              _U32, _U32, _U32]),
         "h3_gpu_fill_normal_bf16": (_I, [_P, _P, _SZ, _SZ, C.c_uint64, _F,
                                          _F]),
         "h3_gpu_fill_normal_f32": (_I, [_P, _P, _SZ, _SZ, C.c_uint64, _F,

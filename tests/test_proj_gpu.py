@@ -2,6 +2,9 @@
 import numpy as np
 import pytest
 
+import oracle
+from conftest import to_f32
+
 pytestmark = pytest.mark.gpu
 
 
@@ -44,3 +47,43 @@ def test_linear_f32_nonfinite(gpu):
     got = gpu.read_f32(out).reshape(m, n)
     want = x @ w.T
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("rows,k,n,mapped", [
+    (1, 4, 4, False), (63, 12, 124, False), (64, 32, 128, True),
+    (65, 36, 132, True), (130, 96, 5376, False), (33, 100, 260, True),
+    (74, 32, 5376, False),
+    (9, 6, 8, False), (9, 8, 6, False),  # K % 4, N % 4: the general kernel
+])
+def test_patch_linear_tiles_bit_exact(gpu, rows, k, n, mapped):
+    """Bit for bit the sequential fmaf order, through every tile edge, from
+    an offset input into an offset output, with values whose products
+    overflow, vanish and cancel."""
+    rng = np.random.default_rng(rows + k + n)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x *= np.exp2(rng.integers(-75, 66, (rows, k))).astype(np.float32)
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    w *= np.exp2(rng.integers(-75, 66, (n, k))).astype(np.float32)
+    b = rng.standard_normal(n).astype(np.float32)
+    out_rows = rows + 7
+    tx, tw, tb = gpu.f32(np.r_[np.zeros(4, np.float32), x.ravel()]), \
+        gpu.f32(w), gpu.f32(b)
+    if mapped:
+        rm = rng.permutation(out_rows)[:rows].astype(np.uint32)
+        out = gpu.bf16(np.full(out_rows * n, 7, np.uint16))
+        gpu.run("h3_hip_patch_linear_bf16_map", out, gpu.f32(x), tw, tb,
+                gpu.u32(rm), out_rows, rows, k, n)
+    else:
+        rm = np.arange(3, 3 + rows, dtype=np.uint32)
+        out = gpu.bf16(np.full(out_rows * n, 7, np.uint16))
+        gpu.run("h3_hip_patch_linear_bf16_offset", out, 3 * n, tx, 4, tw, tb,
+                rows, k, n)
+    got = gpu.read_bf16(out).reshape(out_rows, n)
+    want = oracle.patch_linear(x.ravel(), w.ravel(), b, rows, k, n,
+                               row_map=rm, out_rows=out_rows)
+    want = want.reshape(out_rows, n)
+    nan = np.isnan(to_f32(want))
+    np.testing.assert_array_equal(np.isnan(to_f32(got[rm])), nan[rm])
+    np.testing.assert_array_equal(got[rm][~nan[rm]], want[rm][~nan[rm]])
+    rest = np.setdiff1d(np.arange(out_rows), rm)
+    assert (got[rest] == 7).all()
