@@ -187,4 +187,13 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
                      const uint32_t *row_map, uint32_t m, uint32_t n,
                      uint32_t k);
 
+/* The final adaLN head: RMS adaLN rows, rounded to bf16, times w^T (+ bias),
+ * and each row's inverse RMS; false as above. */
+bool hk_adaln_head(struct h3_gpu *gpu, const uint16_t *x, float *inverse,
+                   const uint16_t *norm, const uint16_t *mod,
+                   const uint32_t *row_map, const uint16_t *w,
+                   const uint16_t *bias, uint16_t *out, uint32_t rows,
+                   uint32_t width, uint32_t n, uint32_t slots,
+                   uint32_t shift_slot, uint32_t scale_slot, float epsilon);
+
 #endif

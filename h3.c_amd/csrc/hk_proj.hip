@@ -1,5 +1,5 @@
 /* Small projections of the DiT path on the matrix cores: the F32 linears of
- * the timestep MLP and the F32 patch projections.
+ * the timestep MLP, the F32 patch projections and the final adaLN heads.
  *
  * F32 MFMAs (v_mfma_f32_16x16x4_f32) multiply and add in full F32: measured
  * on the card, each of their k steps is one fmaf of the accumulator, in k
@@ -272,5 +272,258 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
                             (m + HK_PL_ROWS - 1) / HK_PL_ROWS),
                        dim3(256), 0, gpu->stream, x, w, bias, out, row_map, m,
                        n, k);
+    return true;
+}
+
+/* ------------------------------------------------------ final adaLN head
+ *
+ * RMS adaLN of a row, rounded to bf16, times a [N, width] weight (reference
+ * h3_cuda_dit.cu:183-234).  One workgroup per row had each row read the
+ * whole weight (1 MiB for 96 x 5376) with 2-byte loads.
+ *
+ * Here a workgroup of sixteen waves takes ROWS rows and 16 NB columns.  Each
+ * thread keeps its 8 columns of all the rows in registers, so x is read once
+ * and the norm weight and (when the rows share a modulation row, as a
+ * target's rows do) the shift and scale once for all of them; the
+ * normalised rows go through LDS half a width at a time (16 rows of 5376
+ * are 168 KiB) to be MFMA operands (v_mfma_f32_16x16x32_bf16), and the waves
+ * split the half's 32-wide k steps, reading weight rows from L2.
+ *
+ * A CU takes 64 bytes a clock from its L1, which bounds this kernel: 0.7 MiB
+ * a workgroup with NB = 3 (half of it weights).  Loading x, norm, shift and
+ * scale as MFMA fragments instead (16 lanes repeating each modulation piece)
+ * took 41-44 us at 1792 rows x 96 outputs and 21 us at 74 rows x 32; this
+ * takes 28.7 and 16.7 us.  One workgroup per row: 563 and 198. */
+enum { HK_HEAD_WAVES = 16 };
+
+struct hk_head_args {
+    const uint16_t *x, *norm, *mod, *w, *bias;
+    const uint32_t *row_map;
+    float *inverse;
+    uint16_t *out;
+    uint32_t rows, width, n, slots, shift_slot, scale_slot;
+    float epsilon;
+};
+
+/* bytes of a normalised row's half in LDS: 16 more than its data, so that
+ * the 16 rows of a fragment read start on different banks */
+static __host__ __device__ uint32_t hk_head_pitch(uint32_t width) {
+    return (width / 32u + 1u) / 2u * 64u + 16u;
+}
+
+template <int NB, int ROWS>
+__global__ void __launch_bounds__(HK_HEAD_WAVES * 64)
+hk_adaln_head_mfma(hk_head_args a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t hk_head_lds[];
+    __shared__ float squares[HK_HEAD_WAVES][ROWS];
+    __shared__ float inverses[ROWS];
+    /* weight steps in flight: as many as the registers hold */
+    constexpr uint32_t AHEAD = NB * ROWS > 32 ? 2 : 3;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r16 = lane & 15u, quad = lane >> 4;
+    const uint32_t row0 = blockIdx.x * ROWS;
+    const uint32_t n0 = blockIdx.y * (16u * NB);
+    const uint32_t steps = a.width / 32u, half_steps = (steps + 1u) / 2u;
+    const uint32_t pitch = hk_head_pitch(a.width);
+    const uint32_t col = tid * 8u;
+    const bool mine = col < a.width;
+    /* rows past the end repeat the last one; their outputs are dropped */
+    auto row_of = [&](uint32_t r) { return min(row0 + r, a.rows - 1u); };
+    const uint32_t at = min(col, a.width - 8u); /* loads without a branch */
+    uint4 xv[ROWS];
+#pragma unroll
+    for (uint32_t r = 0; r < ROWS; r++)
+        xv[r] = *(const uint4 *)(a.x + (size_t)row_of(r) * a.width + at);
+    /* ROWS sums over the wave's 64 lanes: each exchange halves the rows a
+     * lane carries, so that the lane's top bits end up naming the row; the
+     * other bits are summed as usual */
+    float sum[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        float v[8];
+        hk_unpack8(xv[r], v);
+        sum[r] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) sum[r] = fmaf(v[e], v[e], sum[r]);
+        if (!mine) sum[r] = 0.0f;
+    }
+#pragma unroll
+    for (int width = ROWS / 2, bit = 32; width; width >>= 1, bit >>= 1)
+#pragma unroll
+        for (int r = 0; r < width; r++) {
+            const bool high = lane & bit;
+            const float keep = high ? sum[r + width] : sum[r];
+            const float send = high ? sum[r] : sum[r + width];
+            sum[r] = keep + __shfl_xor(send, bit, 64);
+        }
+#pragma unroll
+    for (int bit = 32 / ROWS; bit; bit >>= 1)
+        sum[0] += __shfl_xor(sum[0], bit, 64);
+    constexpr uint32_t SPAN = 64 / ROWS; /* lanes that hold one row's sum */
+    if (lane % SPAN == 0) squares[wave][lane / SPAN] = sum[0];
+    /* x stays packed until it is normalised (unpacked, it spilled) */
+#pragma unroll
+    for (int r = 0; r < ROWS; r++)
+        asm volatile("" : "+v"(xv[r].x), "+v"(xv[r].y), "+v"(xv[r].z),
+                          "+v"(xv[r].w));
+    __syncthreads();
+    if (tid < ROWS) {
+        float total = 0.0f;
+#pragma unroll
+        for (int v = 0; v < HK_HEAD_WAVES; v++) total += squares[v][tid];
+        const float inverse =
+            1.0f / sqrtf(total / (float)a.width + a.epsilon);
+        inverses[tid] = inverse;
+        if (blockIdx.y == 0 && row0 + tid < a.rows)
+            a.inverse[row0 + tid] = inverse;
+    }
+    const uint4 nw = *(const uint4 *)(a.norm + at);
+    uint4 sh, sc;
+    auto load_mod = [&](uint32_t map) {
+        const uint16_t *mod = a.mod + (size_t)map * a.slots * a.width + at;
+        sh = *(const uint4 *)(mod + (size_t)a.shift_slot * a.width);
+        sc = *(const uint4 *)(mod + (size_t)a.scale_slot * a.width);
+    };
+    /* readfirstlane: a branch on the map must not become a lane mask */
+    uint32_t map = __builtin_amdgcn_readfirstlane(a.row_map[row_of(0)]);
+    load_mod(map);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < ROWS; r++) {
+        const uint32_t next =
+            __builtin_amdgcn_readfirstlane(a.row_map[row_of(r)]);
+        if (next != map) {
+            map = next;
+            load_mod(map);
+        }
+        /* opaque at both ends: many unpacked rows at a time would spill */
+        asm volatile("" : "+v"(xv[r].x), "+v"(xv[r].y), "+v"(xv[r].z),
+                          "+v"(xv[r].w));
+        const float inverse = inverses[r];
+        float v[8], w8[8], s8[8], c8[8], y[8];
+        hk_unpack8(xv[r], v);
+        hk_unpack8(nw, w8);
+        hk_unpack8(sh, s8);
+        hk_unpack8(sc, c8);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float n = v[e] * inverse * w8[e];
+            y[e] = n * (1.0f + c8[e]) + s8[e];
+        }
+        xv[r] = hk_pack8(y);
+        asm volatile("" : "+v"(xv[r].x), "+v"(xv[r].y), "+v"(xv[r].z),
+                          "+v"(xv[r].w));
+    }
+    /* weight rows past N repeat the last one; those columns are dropped */
+    const uint16_t *wr[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        wr[b] = a.w + (size_t)min(n0 + 16u * b + r16, a.n - 1u) * a.width +
+                quad * 8u;
+    hk_f32x4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[b] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (uint32_t h = 0; h < 2; h++) {
+        const uint32_t first = h * half_steps;
+        const uint32_t count = h ? steps - half_steps : half_steps;
+        if (h) __syncthreads(); /* the first half has been read */
+        if (mine && col / 32u >= first && col / 32u < first + count) {
+            uint8_t *dst = hk_head_lds + (col - first * 32u) * 2u;
+#pragma unroll
+            for (uint32_t r = 0; r < ROWS; r++)
+                *(uint4 *)(dst + r * pitch) = xv[r];
+        }
+        /* AHEAD steps' weights in flight, the first ones across the
+         * barrier; steps past the half repeat its last one */
+        hk_bf16x8 wf[AHEAD][NB];
+        auto load = [&](uint32_t s0) {
+#pragma unroll
+            for (uint32_t u = 0; u < AHEAD; u++)
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    wf[u][b] = *(const hk_bf16x8 *)(
+                        wr[b] +
+                        (first + min(s0 + u * HK_HEAD_WAVES, count - 1u)) *
+                            32u);
+        };
+        if (wave < count) load(wave);
+        __syncthreads();
+        for (uint32_t s0 = wave; s0 < count; s0 += AHEAD * HK_HEAD_WAVES) {
+#pragma unroll
+            for (uint32_t u = 0; u < AHEAD; u++) {
+                const uint32_t s = s0 + u * HK_HEAD_WAVES;
+                if (s >= count) break;
+                const hk_bf16x8 xf = *(const hk_bf16x8 *)(
+                    hk_head_lds + (r16 % ROWS) * pitch + s * 64u +
+                    quad * 16u);
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        wf[u][b], xf, acc[b], 0, 0, 0);
+            }
+            if (s0 + AHEAD * HK_HEAD_WAVES < count)
+                load(s0 + AHEAD * HK_HEAD_WAVES);
+        }
+    }
+    __syncthreads();
+    /* acc[b][i] = out[row0 + r16][n0 + 16 b + 4 quad + i], summed over the
+     * waves in wave order */
+    hk_f32x4 *red = (hk_f32x4 *)hk_head_lds;
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        red[(wave * NB + b) * 64u + lane] = acc[b];
+    __syncthreads();
+    if (tid >= NB * 64u || r16 >= ROWS || row0 + r16 >= a.rows) return;
+    hk_f32x4 total = red[tid];
+#pragma unroll
+    for (int v = 1; v < HK_HEAD_WAVES; v++) total += red[v * NB * 64u + tid];
+    const uint32_t c = n0 + (tid >> 6) * 16u + quad * 4u;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (c + i < a.n)
+            a.out[(size_t)(row0 + r16) * a.n + c + i] = hk_f2bf(
+                a.bias ? total[i] + hk_bf2f(a.bias[c + i]) : total[i]);
+}
+
+template <int NB, int ROWS>
+static void hk_head_run(struct h3_gpu *gpu, const hk_head_args &a) {
+    const size_t tile = (size_t)ROWS * hk_head_pitch(a.width);
+    const size_t sums = (size_t)HK_HEAD_WAVES * NB * 64 * sizeof(hk_f32x4);
+    const size_t lds = tile > sums ? tile : sums;
+    (void)hipFuncSetAttribute((const void *)hk_adaln_head_mfma<NB, ROWS>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)lds);
+    hipLaunchKernelGGL((hk_adaln_head_mfma<NB, ROWS>),
+                       dim3((a.rows + ROWS - 1) / ROWS,
+                            (a.n + 16 * NB - 1) / (16 * NB)),
+                       dim3(HK_HEAD_WAVES * 64), lds, gpu->stream, a);
+}
+
+bool hk_adaln_head(struct h3_gpu *gpu, const uint16_t *x, float *inverse,
+                   const uint16_t *norm, const uint16_t *mod,
+                   const uint32_t *row_map, const uint16_t *w,
+                   const uint16_t *bias, uint16_t *out, uint32_t rows,
+                   uint32_t width, uint32_t n, uint32_t slots,
+                   uint32_t shift_slot, uint32_t scale_slot, float epsilon) {
+    /* a thread per 8 columns, loaded 16 bytes at a time */
+    if (width % 32 || width > HK_HEAD_WAVES * 64 * 8 || !n ||
+        n > 65535u * 32u || ((uintptr_t)x & 15) || ((uintptr_t)norm & 15) ||
+        ((uintptr_t)mod & 15) || ((uintptr_t)w & 15))
+        return false;
+    const hk_head_args a = {x,       norm, mod, w,     bias,  row_map,
+                            inverse, out,  rows, width, n,    slots,
+                            shift_slot, scale_slot, epsilon};
+    /* 4 rows a workgroup while one round of workgroups covers them (16.7 us
+     * against 22.0 with 16 at 74 rows x 32, where a workgroup's own chain of
+     * steps is all that counts), else 16, which read the weights a quarter
+     * as often */
+    const uint32_t groups = n <= 32 ? 1u : (n + 47u) / 48u;
+    const bool few = (rows + 3u) / 4u * groups <= (uint32_t)gpu->num_cus;
+    if (n <= 32 && few) hk_head_run<2, 4>(gpu, a);
+    else if (n <= 32) hk_head_run<2, 16>(gpu, a);
+    else if (few) hk_head_run<3, 4>(gpu, a);
+    else hk_head_run<3, 16>(gpu, a);
     return true;
 }

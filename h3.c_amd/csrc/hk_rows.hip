@@ -2263,7 +2263,13 @@ int h3_gpu_adaln_linear_bf16(h3_gpu *gpu, h3_gpu_tensor *output,
     if ((size_t)width * sizeof(float) > 64 * 1024)
         return hk_fail(gpu, "fused final head width is too large");
     hk_op_begin(gpu, "adaln_head");
-    if (rows && width)
+    if (rows && width &&
+        !hk_adaln_head(gpu, HK_CBF16(input) + input_offset, HK_F32(inverse),
+                       HK_CBF16(norm_weight), HK_CBF16(modulation),
+                       HK_CU32(row_map), HK_CBF16(weight),
+                       bias ? HK_CBF16(bias) : (const uint16_t *)NULL,
+                       HK_BF16(output), rows, width, output_dim, slots,
+                       shift_slot, scale_slot, epsilon))
         hipLaunchKernelGGL(hk_adaln_head_kernel, dim3(rows), dim3(256),
                            width * sizeof(float), gpu->stream,
                            HK_CBF16(input) + input_offset, HK_F32(inverse),

@@ -1,9 +1,11 @@
 """The small projections on the matrix cores, at the edges of their tiles."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle
-from conftest import to_f32
+from conftest import assert_close, rand_bf16, to_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +89,35 @@ def test_patch_linear_tiles_bit_exact(gpu, rows, k, n, mapped):
     np.testing.assert_array_equal(got[rm][~nan[rm]], want[rm][~nan[rm]])
     rest = np.setdiff1d(np.arange(out_rows), rm)
     assert (got[rest] == 7).all()
+
+
+@pytest.mark.parametrize("rows,width,n", [
+    (1, 32, 1), (16, 256, 32), (17, 288, 33), (31, 6144, 96), (5, 5376, 95),
+    (33, 5376, 32), (3, 512, 97), (2, 8192, 48),
+    (1025, 64, 32), (517, 96, 33),  # 16 rows a workgroup
+    (4, 8224, 96), (4, 264, 8),  # the general kernel
+])
+@pytest.mark.parametrize("shared", [True, False])
+def test_adaln_head_tiles(gpu, rows, width, n, shared):
+    """The head against the oracle through its row, width and column edges:
+    one bf16 flip of a normalised value moves an output by 2^-8 of one
+    product, the composite bound of assert_close."""
+    rng = np.random.default_rng(rows + width + n)
+    slots, mods = 3, 4
+    x = rand_bf16(rng, (rows + 2) * width)
+    nw = rand_bf16(rng, width, 0.1, 1.0)
+    mod = rand_bf16(rng, mods * slots * width, 0.2)
+    rm = rng.integers(0, mods, rows).astype(np.uint32)
+    if shared:
+        rm[:] = 2
+    w, b = rand_bf16(rng, n * width, 0.05), rand_bf16(rng, n, 0.1)
+    for bias in (b, None):
+        want, inv = oracle.adaln_linear(x[2 * width:], nw, mod, rm, w, bias,
+                                        rows, width, n, slots, 2, 0, 1e-5)
+        out, tinv = gpu.new_bf16(rows * n), gpu.new_f32(rows)
+        gpu.run("h3_gpu_adaln_linear_bf16", out, tinv, gpu.bf16(x), 2 * width,
+                gpu.bf16(nw), gpu.bf16(mod), gpu.u32(rm), gpu.bf16(w),
+                None if bias is None else gpu.bf16(bias), rows, width, n,
+                slots, 2, 0, C.c_float(1e-5))
+        np.testing.assert_allclose(gpu.read_f32(tinv), inv, rtol=1e-5)
+        assert_close(gpu.read_bf16(out), want, what="head", chained=1)
