@@ -66,6 +66,10 @@
 /* + 256 bytes that the L2 prefetch loads write and nothing reads */
 #define HK_GEMM_LDS (HK_STAGES * HK_STAGE_BYTES + 256) /* 128 KiB + 256 */
 #define HK_GROUP_M 8
+/* rows the skinny GEMM takes: four 32-row MFMA blocks */
+#define HK_SKINNY_ROWS 128u
+/* its operands' bytes stay below this bit, which marks a dead offset */
+#define HK_SKINNY_LIMIT 0x80000000u
 
 typedef int hk_v4i __attribute__((ext_vector_type(4)));
 typedef int hk_v2i __attribute__((ext_vector_type(2)));
@@ -261,65 +265,99 @@ extern "C" int h3_hip_gemm_trace_read(uint64_t *out, size_t entries) {
 }
 #endif
 
-/* Skinny GEMM for M <= 64 rows (the per-block modulation projections:
- * time rows x 2688 against 96768 x 2688 weights).  Bound by streaming W
- * from HBM once, and W is never re-read: each wave owns 32 W rows (output
- * columns) and loads them into registers D - 1 64-wide k steps ahead of
- * the MFMAs, as whole 128-byte lines (a load gives lane l chunk l % 8 of
- * row 8 q + l / 8: eight rows per load, where loading the MFMA fragments
- * directly touches 32 partial rows per load and runs into the cache-line
- * request rate, 27% slower).  The lines go through the wave's own 4-KiB
- * LDS buffer (row-major, the big GEMM's chunk swizzle) and come back out
- * as MFMA fragments.  X (MB x 32 rows) is shared by the workgroup's four
- * waves:
- * one DMA load per thread and step stages it into LDS (double-buffered,
- * 128-byte rows with the 16-byte-chunk swizzle of the big GEMM), so L2
- * serves it once per workgroup instead of once per wave.  The step's k
- * offset goes in the buffer's scalar offset; rows past M or N keep a lane
- * offset beyond the buffer and read zeros.
+/* Skinny GEMM for M <= 128 rows (the per-block modulation projections: time
+ * rows x 2688 against 96768 x 2688 weights; the text refiner's projections of
+ * a short prompt).  Bound by streaming W from HBM once, and W is never
+ * re-read: each wave owns 32 W rows (output columns) and loads them into
+ * registers D - 1 64-wide k steps ahead of the MFMAs, as whole 128-byte lines
+ * (a load gives lane l chunk l % 8 of row 8 q + l / 8: eight rows per load,
+ * where loading the MFMA fragments directly touches 32 partial rows per load
+ * and runs into the cache-line request rate, 27% slower).  The lines go
+ * through the wave's own 4-KiB LDS buffer (row-major, the big GEMM's chunk
+ * swizzle) and come back out as MFMA fragments.  X (MB x 32 rows) is shared
+ * by the workgroup's four waves: MB DMA loads per thread and step stage it
+ * into LDS, XA steps ahead in a ring of XA + 1 stages (128-byte rows with the
+ * 16-byte-chunk swizzle of the big GEMM), so L2 serves it once per workgroup
+ * instead of once per wave.  The step's k offset goes in the buffer's scalar
+ * offset; rows past M or N keep a lane offset beyond the buffer and read
+ * zeros.
  *
- * Ordering: the prologue issues W(0), W(1), X(0), W(2); step s waits until
- * at most the 4 loads of W(s+2) are outstanding (loads retire in order, so
- * X(s) and W(s) have landed), synchronises, stages X(s+1) into the buffer
- * every wave finished reading in step s-1, issues W(s+3) and computes. */
+ * XA = 3 hides X's L2 latency behind two steps: with one stage ahead every
+ * step waited for it where a CU has only one or two workgroups (40 rows x
+ * 5376 -> 21504, 168 workgroups: 48.4 us against 56; 120 rows: 65 against
+ * 94).  With three rounds of workgroups and 64 rows or fewer, XA = 1 is
+ * 3-4% ahead (39 rows x 2688 -> 96768: 96.6 us against 100): its smaller
+ * LDS lets more workgroups share a CU.
+ *
+ * Where one workgroup per 128 columns leaves CUs idle, K is split into as
+ * many pieces as there are CUs for (blockIdx.y), which write F32 sums that
+ * hk_skinny_reduce adds: 8 x 14336 -> 5376 takes 32 us instead of 146, 120
+ * rows 45 instead of 231.  Two workgroups a CU were slower on all but one
+ * shape (34 us, 45-53 us): each piece pays its own start and its sums.
+ *
+ * Ordering: a step waits until X(s) has landed (loads retire in order; W(s)
+ * is a register result the compiler waits for), synchronises, stages
+ * X(s + XA) into the buffer every wave finished reading in step s - 1, issues
+ * W(s + 3) and computes. */
 /* One 64-wide k step of X rows into an LDS stage: thread tid's MB
  * direct-to-LDS loads fill slots 256 i + tid. */
 template <int MB>
 __device__ __forceinline__ void hk_skinny_stage_x(
     __amdgpu_buffer_rsrc_t xr, uint8_t *stage, const uint32_t *xo,
-    uint32_t wave, uint32_t step) {
+    uint32_t wave, uint32_t step, uint32_t dead) {
 #pragma unroll
     for (int i = 0; i < MB; i++)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             xr,
             (__attribute__((address_space(3))) void *)(
                 stage + (256u * i + wave * 64u) * 16u),
-            16, xo[i], step * 128u, 0, 0);
+            16, xo[i] | dead, step * 128u, 0, 0);
 }
 
-template <int MB>
+struct hk_skinny_args {
+    const uint16_t *x, *w, *bias;
+    uint16_t *c;
+    uint32_t m, n, k, x_bytes, w_bytes;
+    /* split-K: workgroup (.., y) takes k steps [y split_steps, + split_steps)
+     * and writes F32 sums to partial[y][32-column tile][MB][4][64 lanes] */
+    float *partial;
+    uint32_t split_steps;
+    /* problem blockIdx.z's W, bias and C (a grouped launch), or null */
+    const uint64_t *group;
+};
+
+template <int MB, int XA>
 __global__ void __launch_bounds__(256)
-hk_gemm_skinny(const uint16_t *x, const uint16_t *w, const uint16_t *bias,
-               uint16_t *c, uint32_t m, uint32_t n, uint32_t k,
-               uint32_t x_bytes, uint32_t w_bytes) {
+hk_gemm_skinny(hk_skinny_args g) {
+    const uint32_t n = g.n, m = g.m, k = g.k;
+    const uint16_t *w = g.w, *bias = g.bias;
+    uint16_t *c = g.c;
+    if (g.group) {
+        w = (const uint16_t *)hk_group_word(g.group, 3 * blockIdx.z);
+        bias = (const uint16_t *)hk_group_word(g.group, 3 * blockIdx.z + 1);
+        c = (uint16_t *)hk_group_word(g.group, 3 * blockIdx.z + 2);
+    }
+    /* k steps of this split; its byte offset goes in the scalar offsets */
+    const uint32_t base = g.partial ? blockIdx.y * g.split_steps : 0u;
+    const uint32_t steps =
+        g.partial ? min(g.split_steps, k / 64u - base) : k / 64u;
     constexpr int D = 4;
     constexpr uint32_t XSTAGE = MB * 32u * 128u; /* bytes of X per k step */
-    /* two X stages (2 XSTAGE bytes), then the four waves' 4-KiB W buffers:
-     * 2 XSTAGE + 16 KiB of dynamic LDS */
+    /* XA + 1 X stages, then the four waves' 4-KiB W buffers */
     extern __shared__ __attribute__((aligned(16))) uint8_t hk_xs[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t row = lane & 31u, half = lane >> 5;
     const uint32_t n0 = (blockIdx.x * 4u + wave) * 32u;
-    const __amdgpu_buffer_rsrc_t xr = hk_rsrc(x, x_bytes);
-    const __amdgpu_buffer_rsrc_t wr = hk_rsrc(w, w_bytes);
+    const __amdgpu_buffer_rsrc_t xr = hk_rsrc(g.x, g.x_bytes);
+    const __amdgpu_buffer_rsrc_t wr = hk_rsrc(w, g.w_bytes);
     uint32_t wo[4];
 #pragma unroll
     for (int q = 0; q < 4; q++)
         wo[q] = (min(n0 + 8u * q + (lane >> 3), n) * k + (lane & 7u) * 8u) *
                 2u;
-    /* the wave's W buffer, after the two X stages */
-    uint8_t *wbuf = hk_xs + 2u * XSTAGE + wave * 4096u;
+    /* the wave's W buffer, after the X stages */
+    uint8_t *wbuf = hk_xs + (XA + 1) * XSTAGE + wave * 4096u;
     /* X staging: slot p = 256 i + tid holds row p / 8, physical chunk p % 8
      * = logical chunk (p % 8) ^ key(row) */
     uint32_t xo[MB];
@@ -329,15 +367,19 @@ hk_gemm_skinny(const uint16_t *x, const uint16_t *w, const uint16_t *bias,
         const uint32_t chunk = (p & 7u) ^ hk_swz_key(r);
         xo[i] = (min(r, m) * k + chunk * 8u) * 2u;
     }
+    auto dead = [&](uint32_t step) {
+        return step < steps ? 0u : HK_SKINNY_LIMIT;
+    };
     auto stage_x = [&](int buf, uint32_t step) {
-        hk_skinny_stage_x<MB>(xr, hk_xs + buf * XSTAGE, xo, wave, step);
+        hk_skinny_stage_x<MB>(xr, hk_xs + buf * XSTAGE, xo, wave, base + step,
+                              dead(step));
     };
     hk_v4i wf[D][4];
     auto load_w = [&](int slot, uint32_t step) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
             wf[slot][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                wr, wo[q], step * 128u, 0);
+                wr, wo[q] | dead(step), (base + step) * 128u, 0);
     };
     /* fragment of X rows mb*32 + row, logical chunk 2q + half */
     auto read_x = [&](int buf, int mb, int q) {
@@ -351,26 +393,29 @@ hk_gemm_skinny(const uint16_t *x, const uint16_t *w, const uint16_t *bias,
     for (int mb = 0; mb < MB; mb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[mb][r] = 0.0f;
-    const uint32_t steps = k / 64u;
-    load_w(0, 0);
-    if (steps > 1) load_w(1, 1);
-    stage_x(0, 0);
-    if (steps > 2) load_w(2, 2);
+    /* Steps past the end load zeros (offsets beyond the buffers, no memory
+     * touched) and add nothing, so the loop has no branch: behind one, the
+     * compiler drains every load in flight. */
+#pragma unroll
+    for (uint32_t d = 0; d + 1 < D; d++) {
+        if (d < XA) stage_x(d, d);
+        load_w(d, d);
+    }
     for (uint32_t s0 = 0; s0 < steps; s0 += D) {
 #pragma unroll
         for (int d = 0; d < D; d++) {
             const uint32_t s = s0 + d;
-            if (s >= steps) break;
-            if (s + 2 < steps)
-                asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-            else
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            /* X(s) has landed: after it, step s - XA issued one W step and
+             * the XA - 1 steps since then MB + 4 loads each */
+            asm volatile("s_waitcnt vmcnt(%0)" ::"i"(
+                             4 + (XA - 1) * (MB + 4))
+                         : "memory");
             /* the barrier as inline assembly: __syncthreads() would also
-             * wait for every load in flight (vmcnt(0)), the W loads of the
+             * wait for every load in flight (vmcnt(0)), the loads of the
              * steps ahead included */
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (s + 1 < steps) stage_x((d + 1) & 1, s + 1);
-            if (s + 3 < steps) load_w((d + 3) % D, s + 3);
+            stage_x((d + XA) % (XA + 1), s + XA);
+            load_w((d + 3) % D, s + 3);
             /* W(s)'s lines into the wave's buffer and back out as
              * fragments (a wave's LDS operations run in order: no
              * barrier) */
@@ -392,10 +437,28 @@ hk_gemm_skinny(const uint16_t *x, const uint16_t *w, const uint16_t *bias,
                 for (int mb = 0; mb < MB; mb++)
                     acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                         __builtin_bit_cast(hk_bf16x8, wfrag[q]),
-                        read_x(d & 1, mb, q), acc[mb], 0, 0, 0);
+                        read_x(d % (XA + 1), mb, q), acc[mb], 0, 0, 0);
         }
     }
     /* acc[mb][r] = C[mb*32 + row][n0 + (r/4)*8 + half*4 + r%4] */
+    if (g.partial) {
+        /* whole lines: each (mb, q) is a wave's 64 16-byte pieces */
+        hk_f32x4 *part =
+            (hk_f32x4 *)g.partial +
+            ((size_t)blockIdx.y * gridDim.x * 4u + blockIdx.x * 4u + wave) *
+                (MB * 256u);
+        if (n0 >= n) return;
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            if (mb * 32u + row >= m) continue;
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                part[(mb * 4u + q) * 64u + lane] =
+                    hk_f32x4{acc[mb][q * 4], acc[mb][q * 4 + 1],
+                             acc[mb][q * 4 + 2], acc[mb][q * 4 + 3]};
+        }
+        return;
+    }
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
         const uint32_t mm = mb * 32u + row;
@@ -418,6 +481,33 @@ hk_gemm_skinny(const uint16_t *x, const uint16_t *w, const uint16_t *bias,
                 uint2{hk_pack2(out[0], out[1]), hk_pack2(out[2], out[3])};
         }
     }
+}
+
+/* Sums the split-K partials of hk_gemm_skinny, in split order, adds the bias
+ * and rounds: one thread per 4 output columns. */
+__global__ void __launch_bounds__(256)
+hk_skinny_reduce(hk_skinny_args g, uint32_t mbs, uint32_t tiles,
+                 uint32_t splits) {
+    /* blockIdx.x = tile * mbs + mb; threads run over (q, lane) */
+    const uint32_t lane = threadIdx.x & 63u, q = threadIdx.x >> 6;
+    const uint32_t tile = blockIdx.x / mbs, mb = blockIdx.x % mbs;
+    const uint32_t row = mb * 32u + (lane & 31u);
+    const uint32_t col = tile * 32u + q * 8u + (lane >> 5) * 4u;
+    if (row >= g.m || col >= g.n) return;
+    const hk_f32x4 *p = (const hk_f32x4 *)g.partial +
+                        (size_t)blockIdx.x * 256u + threadIdx.x;
+    const size_t stride = (size_t)tiles * mbs * 256u;
+    hk_f32x4 sum = *p;
+    for (uint32_t s = 1; s < splits; s++) sum += p[s * stride];
+    if (g.bias) {
+        const uint2 b = *(const uint2 *)(g.bias + col);
+        sum[0] += hk_bf2f(b.x & 0xffffu);
+        sum[1] += hk_bf2f(b.x >> 16);
+        sum[2] += hk_bf2f(b.y & 0xffffu);
+        sum[3] += hk_bf2f(b.y >> 16);
+    }
+    *(uint2 *)(g.c + (size_t)row * g.n + col) =
+        make_uint2(hk_pack2(sum[0], sum[1]), hk_pack2(sum[2], sum[3]));
 }
 
 /* Sequential-k reference GEMM (any shape).  For SwiGLU it writes the fused
@@ -587,6 +677,75 @@ static void hk_gemm_lds_setup(const struct h3_gpu *gpu) {
     hk_gemm_lds_ready |= bit;
 }
 
+/* Whether a shape that hk_gemm_mfma_ok takes is one for hk_gemm_skinny. */
+static bool hk_skinny_ok(uint32_t m, uint32_t n, uint32_t k) {
+    const uint64_t margin = 4ull * k + 4096;
+    return m <= HK_SKINNY_ROWS &&
+           (uint64_t)n * k * 2 + margin < HK_SKINNY_LIMIT &&
+           (uint64_t)m * k * 2 + margin < HK_SKINNY_LIMIT;
+}
+
+/* 80 KiB of dynamic LDS need the kernel's limit raised, once per device. */
+static void hk_skinny_lds_setup(const struct h3_gpu *gpu) {
+    static uint64_t ready = 0;
+    const uint64_t bit = 1ull << (gpu->device & 63);
+    if (ready & bit) return;
+    (void)hipFuncSetAttribute((const void *)hk_gemm_skinny<4, 3>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              4 * 4096 * 4 + 16384);
+    ready |= bit;
+}
+
+/* Launches hk_gemm_skinny: `problems` of them from a table, or one. */
+static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
+                              const uint16_t *w, const uint16_t *bias,
+                              uint16_t *c, uint32_t m, uint32_t n, uint32_t k,
+                              const uint64_t *group, uint32_t problems,
+                              float *scratch, size_t scratch_bytes) {
+    const uint32_t mbs = (m + 31u) / 32u, wgs = (n + 127u) / 128u;
+    const uint32_t k_steps = k / HK_BK;
+    hk_skinny_args g;
+    g.x = x; g.w = w; g.bias = bias; g.c = c;
+    g.m = m; g.n = n; g.k = k;
+    g.x_bytes = (uint32_t)((uint64_t)m * k * 2);
+    g.w_bytes = (uint32_t)((uint64_t)n * k * 2);
+    g.partial = NULL;
+    g.split_steps = k_steps;
+    g.group = group;
+    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
+    /* one workgroup per CU, pieces of at least two turns of the ring */
+    uint32_t splits = group ? 1u : min(cus / wgs, k_steps / 8u);
+    if (splits > 1) {
+        /* whole turns of the kernel's ring of 4 */
+        g.split_steps = ((k_steps + splits - 1) / splits + 3u) & ~3u;
+        splits = (k_steps + g.split_steps - 1) / g.split_steps;
+    }
+    const size_t bytes = (size_t)splits * wgs * 4 * mbs * 4096;
+    /* at most a 64-KiB piece per CU: a quarter of the no-alloc scratch */
+    if (scratch && bytes > scratch_bytes) splits = 1;
+    if (splits > 1) {
+        g.partial = scratch ? scratch
+                            : (float *)hk_splitk_space(gpu, bytes);
+        if (!g.partial) return 0;
+    }
+    const dim3 grid(wgs, splits > 1 ? splits : 1u, problems);
+    /* several rounds of few rows: one X stage ahead (both timed above) */
+    const int ahead = mbs <= 2 && wgs * problems >= 2 * cus ? 1 : 3;
+    const size_t lds = mbs * 4096 * (ahead + 1) + 16384;
+    void (*kernel)(hk_skinny_args) =
+        mbs == 1   ? (ahead == 1 ? hk_gemm_skinny<1, 1> : hk_gemm_skinny<1, 3>)
+        : mbs == 2 ? (ahead == 1 ? hk_gemm_skinny<2, 1> : hk_gemm_skinny<2, 3>)
+        : mbs == 3 ? hk_gemm_skinny<3, 3>
+                   : hk_gemm_skinny<4, 3>;
+    if (mbs == 4) hk_skinny_lds_setup(gpu);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, gpu->stream, g);
+    if (g.partial)
+        hipLaunchKernelGGL(hk_skinny_reduce, dim3((n + 31) / 32 * mbs),
+                           dim3(256), 0, gpu->stream, g, mbs, wgs * 4,
+                           splits);
+    return 1;
+}
+
 int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
                  const uint16_t *bias, uint16_t *c, uint32_t m, uint32_t n,
                  uint32_t k, int epilogue, float *scratch,
@@ -595,19 +754,9 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
     const uint64_t w_rows = epilogue == HK_EPI_SWIGLU ? 2ull * n : n;
     const uint64_t x_bytes = (uint64_t)m * k * 2, w_bytes = w_rows * k * 2;
     const bool mfma = hk_gemm_mfma_ok(gpu, x, w, bias, c, m, n, k, epilogue);
-    if (mfma && m <= 64 && epilogue == HK_EPI_STORE) {
-        if (m <= 32)
-            hipLaunchKernelGGL(hk_gemm_skinny<1>, dim3((n + 127) / 128),
-                               dim3(256), 2 * 32 * 128 + 16384, gpu->stream, x, w,
-                               bias, c, m, n, k, (uint32_t)x_bytes,
-                               (uint32_t)w_bytes);
-        else
-            hipLaunchKernelGGL(hk_gemm_skinny<2>, dim3((n + 127) / 128),
-                               dim3(256), 2 * 64 * 128 + 16384, gpu->stream, x, w,
-                               bias, c, m, n, k, (uint32_t)x_bytes,
-                               (uint32_t)w_bytes);
-        return 1;
-    }
+    if (mfma && epilogue == HK_EPI_STORE && hk_skinny_ok(m, n, k))
+        return hk_gemm_skinny_run(gpu, x, w, bias, c, m, n, k, NULL, 1,
+                                  scratch, scratch_bytes);
     if (mfma) {
         hk_gemm_lds_setup(gpu);
         hk_gemm_args g;
@@ -744,7 +893,7 @@ int hk_gemm_bf16_pair(struct h3_gpu *gpu, const uint16_t *x,
     const uint32_t tiles = ((m + HK_BM - 1) / HK_BM) * ((n + HK_BN - 1) / HK_BN);
     const uint32_t k_steps = k / HK_BK;
     const bool paired =
-        m > 64 && k_steps >= 8 && tiles * 4 <= cus &&
+        !hk_skinny_ok(m, n, k) && k_steps >= 8 && tiles * 4 <= cus &&
         hk_gemm_mfma_ok(gpu, x, w0, b0, c0, m, n, k, HK_EPI_STORE) &&
         hk_gemm_mfma_ok(gpu, x, w1, b1, c1, m, n, k, HK_EPI_STORE);
     if (!paired)
@@ -789,6 +938,15 @@ static int hk_gemm_bf16_group(struct h3_gpu *gpu, const uint16_t *x,
                               const uint64_t *table, uint32_t count,
                               uint32_t m, uint32_t n, uint32_t k) {
     if (!m || !n || !count) return 1;
+    if (hk_skinny_ok(m, n, k)) {
+        /* a grid's z dimension ends at 65535 */
+        for (uint32_t p = 0; p < count; p += 65535u)
+            if (!hk_gemm_skinny_run(gpu, x, NULL, NULL, NULL, m, n, k,
+                                    table + (size_t)p * 3,
+                                    min(count - p, 65535u), NULL, 0))
+                return 0;
+        return 1;
+    }
     hk_gemm_lds_setup(gpu);
     hk_gemm_args g;
     memset(&g, 0, sizeof(g));
@@ -999,8 +1157,7 @@ int h3_hip_linear_group_bf16(h3_gpu *gpu, const h3_gpu_tensor *table,
         return 0;
     if (!count) return 1;
     const uint64_t *dev = (const uint64_t *)table->data + (size_t)first * 3;
-    const bool mfma = rows > 64 &&
-                      hk_gemm_mfma_ok(gpu, input->data, input->data, NULL,
+    const bool mfma = hk_gemm_mfma_ok(gpu, input->data, input->data, NULL,
                                       input->data, rows, output_dim,
                                       input_dim, HK_EPI_STORE);
     hk_op_begin(gpu, "gemm_group");
