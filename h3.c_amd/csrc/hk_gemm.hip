@@ -6,7 +6,8 @@
  * of one row, i.e. one 16-byte LDS read per lane.
  *
  * Tiling (per 256-thread workgroup, one workgroup per CU at a time):
- *   - 256 (W rows) x 256 (X rows) output tile, K step 64;
+ *   - 256 (W rows) x 256 (X rows) output tile, K step 64; where 256 rows
+ *     pad too much, 224, 192, 160 or 128 of them (hk_gemm_row_blocks);
  *   - four wave64s in a 2x2 grid, each owning a 128x128 sub-tile held as
  *     8x8 accumulators of v_mfma_f32_16x16x32_bf16 (256 f32 per lane; the
  *     kernel body is in hk_gemm_kernel.inc);
@@ -81,6 +82,26 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t hk_rsrc(const void *base,
                                              0x00020000);
 }
 
+/* A wave's direct-to-LDS loads of 16 or 4 bytes per lane: lane i's bytes go
+ * to lds + 16 i (4 i).  Functions of their own: in a lambda of a kernel
+ * template, the cast to LDS keeps the host pass from emitting the kernel's
+ * launch stub when it depends on the template's parameters. */
+__device__ __forceinline__ void hk_dma16(__amdgpu_buffer_rsrc_t r,
+                                         uint8_t *lds, uint32_t offset,
+                                         uint32_t scalar_offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        r, (__attribute__((address_space(3))) void *)lds, 16, offset,
+        scalar_offset, 0, 0);
+}
+
+__device__ __forceinline__ void hk_dma4(__amdgpu_buffer_rsrc_t r,
+                                        uint8_t *lds, uint32_t offset,
+                                        uint32_t scalar_offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        r, (__attribute__((address_space(3))) void *)lds, 4, offset,
+        scalar_offset, 0, 0);
+}
+
 /* LDS rows are 128 B (64 bf16 = 8 chunks of 16 B); logical chunk c of row
  * r lives at physical chunk c ^ key(r).  Any 8 consecutive rows get
  * distinct keys (32-bank view, 128 B per cycle) and any 16 consecutive rows
@@ -127,11 +148,12 @@ struct hk_gemm_args {
     uint16_t *c;           /* [M, N] */
     uint32_t m, n, k;      /* n = output columns */
     uint32_t tiles_m, tiles_n;
+    uint32_t tile_rows;    /* X rows of a tile: 256, or 32 JB */
     uint32_t x_bytes, w_bytes;
     /* split-K (EPI == HK_EPI_PARTIAL only): workgroup pid covers tile
      * tile_base + pid % part_tiles over K steps [split * split_steps,
      * +split_steps), split = pid / part_tiles, and writes the F32 tile to
-     * partial[split][pid % part_tiles][256][256] */
+     * partial[split][pid % part_tiles][tile_rows][256] */
     float *partial;
     uint32_t split_steps, tile_base, part_tiles;
     /* tiles [0, tile_count) of the launch, dealt to the workgroups in
@@ -233,20 +255,25 @@ __device__ __forceinline__ void hk_trace_put(uint32_t iter, uint32_t slot,
 #define HK_CYCLES() 0ull
 #endif
 
-/* The MFMA shape of the main loop: v_mfma_f32_16x16x32_bf16 for every
- * launch, full tiles and split-K pieces.  At the same 1400 W it runs the
- * GEMM at a higher clock than 32x32x16 (less register-file traffic per
- * flop).  -DHK_MFMA32 builds the kernel with 32x32x16 (4x4 blocks) instead,
- * for comparison. */
+/* The MFMA shape of the main loop is v_mfma_f32_16x16x32_bf16 for every
+ * launch, full tiles and split-K pieces: at the same 1400 W it runs the GEMM
+ * at a higher clock than 32x32x16 (less register-file traffic per flop).
+ * hk_gemm_mfma has 256-row tiles; hk_gemm_mfma_low<.., JB> the same 256
+ * columns and 32 JB rows, for row counts that 256 would pad. */
 #define HK_KERNEL_NAME hk_gemm_mfma
-#ifdef HK_MFMA32
-#define HK_KERNEL_MFMA16 0
-#else
-#define HK_KERNEL_MFMA16 1
-#endif
+#define HK_KERNEL_TEMPLATE template <int EPI, bool GROUP = false>
+#define HK_KERNEL_JB 8
 #include "hk_gemm_kernel.inc"
 #undef HK_KERNEL_NAME
-#undef HK_KERNEL_MFMA16
+#undef HK_KERNEL_TEMPLATE
+#undef HK_KERNEL_JB
+#define HK_KERNEL_NAME hk_gemm_mfma_low
+#define HK_KERNEL_TEMPLATE template <int EPI, bool GROUP, int ROW_BLOCKS>
+#define HK_KERNEL_JB ROW_BLOCKS
+#include "hk_gemm_kernel.inc"
+#undef HK_KERNEL_NAME
+#undef HK_KERNEL_TEMPLATE
+#undef HK_KERNEL_JB
 
 #ifdef HK_GEMM_TRACE
 extern "C" int h3_hip_gemm_trace_clear(void) {
@@ -299,21 +326,6 @@ extern "C" int h3_hip_gemm_trace_read(uint64_t *out, size_t entries) {
  * is a register result the compiler waits for), synchronises, stages
  * X(s + XA) into the buffer every wave finished reading in step s - 1, issues
  * W(s + 3) and computes. */
-/* One 64-wide k step of X rows into an LDS stage: thread tid's MB
- * direct-to-LDS loads fill slots 256 i + tid. */
-template <int MB>
-__device__ __forceinline__ void hk_skinny_stage_x(
-    __amdgpu_buffer_rsrc_t xr, uint8_t *stage, const uint32_t *xo,
-    uint32_t wave, uint32_t step, uint32_t dead) {
-#pragma unroll
-    for (int i = 0; i < MB; i++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            xr,
-            (__attribute__((address_space(3))) void *)(
-                stage + (256u * i + wave * 64u) * 16u),
-            16, xo[i] | dead, step * 128u, 0, 0);
-}
-
 struct hk_skinny_args {
     const uint16_t *x, *w, *bias;
     uint16_t *c;
@@ -371,8 +383,10 @@ hk_gemm_skinny(hk_skinny_args g) {
         return step < steps ? 0u : HK_SKINNY_LIMIT;
     };
     auto stage_x = [&](int buf, uint32_t step) {
-        hk_skinny_stage_x<MB>(xr, hk_xs + buf * XSTAGE, xo, wave, base + step,
-                              dead(step));
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+            hk_dma16(xr, hk_xs + buf * XSTAGE + (256u * i + wave * 64u) * 16u,
+                     xo[i] | dead(step), (base + step) * 128u);
     };
     hk_v4i wf[D][4];
     auto load_w = [&](int slot, uint32_t step) {
@@ -552,17 +566,20 @@ hk_splitk_reduce(hk_gemm_args g, uint32_t splits) {
         /* 8 tile rows per workgroup, 4 output columns per thread: output
          * column c of the tile (128 per tile) is W-tile row (c/64)*128 +
          * c%64 (gate) and that + 64 (up); out = bf16(silu(bf16 g) bf16 u) */
-        const uint32_t part = blockIdx.x >> 5;
-        const uint32_t row = (blockIdx.x & 31u) * 8u + (threadIdx.x >> 5);
+        const uint32_t blocks = g.tile_rows / 8u;
+        const uint32_t part = blockIdx.x / blocks;
+        const uint32_t row =
+            (blockIdx.x - part * blocks) * 8u + (threadIdx.x >> 5);
         const uint32_t c4 = (threadIdx.x & 31u) * 4u;
         uint32_t tile_m, tile_n;
         hk_tile_coords(g.tile_base + part, g.tiles_m, g.tiles_n,
                        tile_m, tile_n);
-        const uint32_t m = tile_m * HK_BM + row, n = tile_n * 128u + c4;
+        const uint32_t m = tile_m * g.tile_rows + row, n = tile_n * 128u + c4;
         if (m >= g.m || n >= g.n) return;
-        const size_t stride = (size_t)g.part_tiles * (HK_BM * HK_BN);
-        const float *p = g.partial + (size_t)part * (HK_BM * HK_BN) +
-                         row * HK_BN + (c4 >> 6) * 128u + (c4 & 63u);
+        const size_t tile = (size_t)g.tile_rows * HK_BN;
+        const size_t stride = g.part_tiles * tile;
+        const float *p = g.partial + part * tile + row * HK_BN +
+                         (c4 >> 6) * 128u + (c4 & 63u);
         float4 gs = *(const float4 *)p, us = *(const float4 *)(p + 64);
         for (uint32_t s = 1; s < splits; s++) {
             const float4 gv = *(const float4 *)(p + s * stride);
@@ -581,20 +598,21 @@ hk_splitk_reduce(hk_gemm_args g, uint32_t splits) {
             make_uint2(hk_pack2(out[0], out[1]), hk_pack2(out[2], out[3]));
         return;
     }
-    const uint32_t part = blockIdx.x >> 6;
-    const uint32_t row = (blockIdx.x & 63u) * 4u + (threadIdx.x >> 6);
+    const uint32_t blocks = g.tile_rows / 4u;
+    const uint32_t part = blockIdx.x / blocks;
+    const uint32_t row = (blockIdx.x - part * blocks) * 4u + (threadIdx.x >> 6);
     const uint32_t tcol = (threadIdx.x & 63u) * 4u;
     const bool second = g.pair_tiles && part >= g.pair_tiles;
     uint32_t tile_m, tile_n;
     hk_tile_coords(g.tile_base + (second ? part - g.pair_tiles : part),
                    g.tiles_m, g.tiles_n, tile_m, tile_n);
-    const uint32_t m = tile_m * HK_BM + row, n = tile_n * HK_BN + tcol;
+    const uint32_t m = tile_m * g.tile_rows + row, n = tile_n * HK_BN + tcol;
     if (m >= g.m || n >= g.n) return;
     const uint16_t *bias = second ? g.bias1 : g.bias;
     uint16_t *c = second ? g.c1 : g.c;
-    const size_t stride = (size_t)g.part_tiles * (HK_BM * HK_BN);
-    const float *p = g.partial + (size_t)part * (HK_BM * HK_BN) +
-                     row * HK_BN + tcol;
+    const size_t tile = (size_t)g.tile_rows * HK_BN;
+    const size_t stride = g.part_tiles * tile;
+    const float *p = g.partial + part * tile + row * HK_BN + tcol;
     float4 sum = *(const float4 *)p;
     for (uint32_t s = 1; s < splits; s++) {
         const float4 v = *(const float4 *)(p + s * stride);
@@ -653,28 +671,135 @@ static bool hk_gemm_mfma_ok(const struct h3_gpu *gpu, const void *x,
            ((uintptr_t)c & 7) == 0 && ((uintptr_t)bias & 7) == 0;
 }
 
+/* The kernel with 32 jb rows per tile, and its dynamic LDS. */
+typedef void (*hk_gemm_kernel)(hk_gemm_args);
+
+template <int EPI, bool GROUP>
+static hk_gemm_kernel hk_gemm_pick(uint32_t jb) {
+    switch (jb) {
+    case 4: return hk_gemm_mfma_low<EPI, GROUP, 4>;
+    case 5: return hk_gemm_mfma_low<EPI, GROUP, 5>;
+    case 6: return hk_gemm_mfma_low<EPI, GROUP, 6>;
+    case 7: return hk_gemm_mfma_low<EPI, GROUP, 7>;
+    default: return hk_gemm_mfma<EPI, GROUP>;
+    }
+}
+
+static hk_gemm_kernel hk_gemm_pick_epi(int epilogue, uint32_t jb) {
+    switch (epilogue) {
+    case HK_EPI_SWIGLU: return hk_gemm_pick<HK_EPI_SWIGLU, false>(jb);
+    case HK_EPI_GELU: return hk_gemm_pick<HK_EPI_GELU, false>(jb);
+    case HK_EPI_PARTIAL: return hk_gemm_pick<HK_EPI_PARTIAL, false>(jb);
+    case HK_EPI_PARTIAL_SWIGLU:
+        return hk_gemm_pick<HK_EPI_PARTIAL_SWIGLU, false>(jb);
+    default: return hk_gemm_pick<HK_EPI_STORE, false>(jb);
+    }
+}
+
+static uint32_t hk_gemm_lds(uint32_t jb) {
+    return HK_STAGES * (32u * jb * HK_BK * 2u + HK_TILE_BYTES) + 256u;
+}
+
 static void hk_gemm_lds_setup(const struct h3_gpu *gpu) {
     const uint64_t bit = 1ull << (gpu->device & 63);
     if (hk_gemm_lds_ready & bit) return;
-    (void)hipFuncSetAttribute((const void *)hk_gemm_mfma<HK_EPI_STORE>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              HK_GEMM_LDS);
-    (void)hipFuncSetAttribute((const void *)hk_gemm_mfma<HK_EPI_SWIGLU>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              HK_GEMM_LDS);
-    (void)hipFuncSetAttribute((const void *)hk_gemm_mfma<HK_EPI_GELU>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              HK_GEMM_LDS);
-    (void)hipFuncSetAttribute((const void *)hk_gemm_mfma<HK_EPI_PARTIAL>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              HK_GEMM_LDS);
-    (void)hipFuncSetAttribute(
-        (const void *)hk_gemm_mfma<HK_EPI_PARTIAL_SWIGLU>,
-        hipFuncAttributeMaxDynamicSharedMemorySize, HK_GEMM_LDS);
-    (void)hipFuncSetAttribute((const void *)hk_gemm_mfma<HK_EPI_STORE, true>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              HK_GEMM_LDS);
+    for (uint32_t jb = 4; jb <= 8; jb++) {
+        for (int epi = HK_EPI_STORE; epi <= HK_EPI_PARTIAL_SWIGLU; epi++)
+            (void)hipFuncSetAttribute(
+                (const void *)hk_gemm_pick_epi(epi, jb),
+                hipFuncAttributeMaxDynamicSharedMemorySize,
+                (int)hk_gemm_lds(jb));
+        (void)hipFuncSetAttribute(
+            (const void *)hk_gemm_pick<HK_EPI_STORE, true>(jb),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)hk_gemm_lds(jb));
+    }
     hk_gemm_lds_ready |= bit;
+}
+
+static void hk_gemm_launch(struct h3_gpu *gpu, hk_gemm_kernel kernel,
+                           uint32_t jb, uint32_t workgroups,
+                           const hk_gemm_args &g) {
+    hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(HK_GEMM_THREADS),
+                       hk_gemm_lds(jb), gpu->stream, g);
+}
+
+/* How the tiles of a launch run: `full` tiles in rounds of one per CU, then
+ * `tail` tiles, cut along K into `splits` pieces of `steps` 64-deep steps when
+ * they would leave over half the CUs idle (splits is 1 otherwise, and the
+ * tail is one more round). */
+struct hk_gemm_rounds {
+    uint32_t full, tail, splits, steps;
+};
+
+static hk_gemm_rounds hk_gemm_rounds_of(uint32_t tiles, uint32_t k_steps,
+                                        uint32_t cus, bool may_split) {
+    hk_gemm_rounds r = {tiles - tiles % cus, tiles % cus, 1, k_steps};
+    if (may_split && r.tail && r.tail * 2 <= cus && k_steps >= 8) {
+        r.splits = min(cus / r.tail, k_steps / 4);
+        r.steps = (k_steps + r.splits - 1) / r.splits;
+        r.splits = (k_steps + r.steps - 1) / r.steps;
+    }
+    return r;
+}
+
+/* Estimated microseconds of a launch of `tiles` tiles of 32 jb rows, fitted
+ * to 630 launches (jb 4-8, 140-6144 rows, seven K x N of the two models, cold
+ * weights; 10% rms): a round's fixed cost, its steps (a quarter faster when
+ * few CUs run and the clock is higher), the pieces' partial sums both ways
+ * through the caches and the reduction. */
+static float hk_gemm_estimate(uint32_t jb, uint32_t tiles, uint32_t k_steps,
+                              uint32_t cus, bool may_split) {
+    static const float step_us[5] = {0.86f, 0.99f, 1.11f, 1.30f, 1.50f};
+    auto round = [&](uint32_t steps, uint32_t workgroups) {
+        const float fill = (float)min(workgroups, cus) / (float)cus;
+        return 12.8f - 0.77f * (float)jb +
+               (float)steps * step_us[jb - 4] * (0.71f + 0.29f * fill);
+    };
+    const hk_gemm_rounds r = hk_gemm_rounds_of(tiles, k_steps, cus, may_split);
+    if (r.splits > 1) {
+        const float partial_mb =
+            (float)(r.splits * r.tail * jb) * (32.0f * HK_BN * 4e-6f);
+        float us = round(r.steps, r.splits * r.tail) + 11.4f +
+                   2.0f * partial_mb / 11.9f;
+        if (r.full) us += (float)(r.full / cus) * round(k_steps, cus) + 6.0f;
+        return us;
+    }
+    const uint32_t rounds = (tiles + cus - 1) / cus;
+    return (float)rounds * round(k_steps, (tiles + rounds - 1) / rounds);
+}
+
+/* The tile height, in 32-row units, for m rows in `columns` column tiles:
+ * the one with the lowest estimate.  256 rows use the fewest cycles and bytes
+ * per flop, but pad 300 rows by 70% and 1300 by 18%, and another height can
+ * fill the last round of CUs: measured (us, 256 rows against the pick) 114
+ * and 100 for 300 x 5376 -> 21504, 190 and 173 for 778 x the same, 145 and
+ * 115 for 1600 x 7168 -> 5376, 316 and 288 for 2378 x 14336 -> 5376.  Where
+ * every tile is split along K, more row tiles read the weights more often
+ * (512 x 14336 -> 5376: 88 us with 256 rows, 121 with 128), which the
+ * estimate leaves out, and 224 rows gained nothing: there only 160 and 192
+ * rows in as many row tiles count. */
+static uint32_t hk_gemm_row_blocks(uint32_t m, uint32_t columns,
+                                   uint32_t k_steps, uint32_t cus,
+                                   bool may_split) {
+    const uint32_t high = (m + HK_BM - 1) / HK_BM;
+    const hk_gemm_rounds r =
+        hk_gemm_rounds_of(high * columns, k_steps, cus, may_split);
+    const bool all_split = r.splits > 1 && !r.full;
+    uint32_t best = 8;
+    /* 1% in favour of the 256-row kernel */
+    float least =
+        0.99f * hk_gemm_estimate(8, high * columns, k_steps, cus, may_split);
+    for (uint32_t jb = 7; jb >= 4; jb--) {
+        const uint32_t tiles_m = (m + 32u * jb - 1) / (32u * jb);
+        if (all_split && (tiles_m > high || jb == 7)) continue;
+        const float us = hk_gemm_estimate(jb, tiles_m * columns, k_steps, cus,
+                                          may_split);
+        if (us < least) {
+            best = jb;
+            least = us;
+        }
+    }
+    return best;
 }
 
 /* Whether a shape that hk_gemm_mfma_ok takes is one for hk_gemm_skinny. */
@@ -762,9 +887,14 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
         hk_gemm_args g;
         g.x = x; g.w = w; g.bias = bias; g.c = c;
         g.m = m; g.n = n; g.k = k;
-        g.tiles_m = (m + HK_BM - 1) / HK_BM;
+        const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
         const uint32_t cols_per_tile = epilogue == HK_EPI_SWIGLU ? 128 : HK_BN;
+        const uint32_t k_steps = k / HK_BK;
         g.tiles_n = (n + cols_per_tile - 1) / cols_per_tile;
+        const uint32_t jb =
+            hk_gemm_row_blocks(m, g.tiles_n, k_steps, cus, true);
+        g.tile_rows = 32u * jb;
+        g.tiles_m = (m + g.tile_rows - 1) / g.tile_rows;
         g.x_bytes = (uint32_t)x_bytes;
         g.w_bytes = (uint32_t)w_bytes;
         g.partial = NULL;
@@ -777,8 +907,6 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
         g.group = NULL;
         g.w1 = g.bias1 = NULL;
         g.c1 = NULL;
-        const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
-        dim3 grid(hk_gemm_grid(g.tile_count, cus));
         /* Split-K for a sparse last round: when the tiles left after the
          * full rounds of one tile per CU (all of them, for small launches
          * like the 512-row cross-attention K/V projections) would leave over
@@ -787,15 +915,13 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
          * adds the F32 partials, the bias and the activation (SwiGLU: the
          * gate and up sums, each rounded to bf16 as the fused epilogue
          * does). */
-        const uint32_t tiles = g.tiles_m * g.tiles_n;
-        const uint32_t k_steps = k / HK_BK;
-        const uint32_t full = tiles - tiles % cus, tail = tiles % cus;
-        if (tail && tail * 2 <= cus && k_steps >= 8) {
-            uint32_t splits = min(cus / tail, k_steps / 4);
-            const uint32_t steps = (k_steps + splits - 1) / splits;
-            splits = (k_steps + steps - 1) / steps;
+        const hk_gemm_rounds r =
+            hk_gemm_rounds_of(g.tile_count, k_steps, cus, true);
+        if (r.splits > 1) {
+            const uint32_t full = r.full, tail = r.tail;
+            const uint32_t splits = r.splits, steps = r.steps;
             const size_t partial_bytes =
-                (size_t)splits * tail * HK_BM * HK_BN * 4;
+                (size_t)splits * tail * g.tile_rows * HK_BN * 4;
             if (scratch && partial_bytes > scratch_bytes)
                 return hk_fail(gpu,
                                "linear needs %zu bytes of split-K scratch, "
@@ -807,58 +933,35 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
             if (!partial) return 0;
             if (full) {
                 g.tile_count = full;
-                const dim3 fgrid(hk_gemm_grid(full, cus));
-                if (epilogue == HK_EPI_GELU)
-                    hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_GELU>, fgrid,
-                                       dim3(HK_GEMM_THREADS), HK_GEMM_LDS,
-                                       gpu->stream, g);
-                else if (epilogue == HK_EPI_SWIGLU)
-                    hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_SWIGLU>, fgrid,
-                                       dim3(HK_GEMM_THREADS), HK_GEMM_LDS,
-                                       gpu->stream, g);
-                else
-                    hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_STORE>, fgrid,
-                                       dim3(HK_GEMM_THREADS), HK_GEMM_LDS,
-                                       gpu->stream, g);
+                hk_gemm_launch(gpu, hk_gemm_pick_epi(epilogue, jb), jb,
+                               hk_gemm_grid(full, cus), g);
             }
             g.partial = partial;
             g.split_steps = steps;
             g.tile_base = full;
             g.part_tiles = tail;
-            if (epilogue == HK_EPI_SWIGLU)
-                hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_PARTIAL_SWIGLU>,
-                                   dim3(tail * splits), dim3(HK_GEMM_THREADS),
-                                   HK_GEMM_LDS, gpu->stream, g);
-            else
-                hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_PARTIAL>,
-                                   dim3(tail * splits), dim3(HK_GEMM_THREADS),
-                                   HK_GEMM_LDS, gpu->stream, g);
+            hk_gemm_launch(gpu,
+                           hk_gemm_pick_epi(epilogue == HK_EPI_SWIGLU
+                                                ? HK_EPI_PARTIAL_SWIGLU
+                                                : HK_EPI_PARTIAL,
+                                            jb),
+                           jb, tail * splits, g);
             if (epilogue == HK_EPI_SWIGLU)
                 hipLaunchKernelGGL(hk_splitk_reduce<HK_EPI_SWIGLU>,
-                                   dim3(tail * 32), dim3(256), 0, gpu->stream,
-                                   g, splits);
+                                   dim3(tail * (g.tile_rows / 8)), dim3(256),
+                                   0, gpu->stream, g, splits);
             else if (epilogue == HK_EPI_GELU)
                 hipLaunchKernelGGL(hk_splitk_reduce<HK_EPI_GELU>,
-                                   dim3(tail * 64), dim3(256), 0, gpu->stream,
-                                   g, splits);
+                                   dim3(tail * (g.tile_rows / 4)), dim3(256),
+                                   0, gpu->stream, g, splits);
             else
                 hipLaunchKernelGGL(hk_splitk_reduce<HK_EPI_STORE>,
-                                   dim3(tail * 64), dim3(256), 0, gpu->stream,
-                                   g, splits);
+                                   dim3(tail * (g.tile_rows / 4)), dim3(256),
+                                   0, gpu->stream, g, splits);
             return 1;
         }
-        if (epilogue == HK_EPI_SWIGLU)
-            hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_SWIGLU>, grid,
-                               dim3(HK_GEMM_THREADS), HK_GEMM_LDS, gpu->stream,
-                               g);
-        else if (epilogue == HK_EPI_GELU)
-            hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_GELU>, grid,
-                               dim3(HK_GEMM_THREADS), HK_GEMM_LDS, gpu->stream,
-                               g);
-        else
-            hipLaunchKernelGGL(hk_gemm_mfma<HK_EPI_STORE>, grid,
-                               dim3(HK_GEMM_THREADS), HK_GEMM_LDS, gpu->stream,
-                               g);
+        hk_gemm_launch(gpu, hk_gemm_pick_epi(epilogue, jb), jb,
+                       hk_gemm_grid(g.tile_count, cus), g);
         return 1;
     }
     if (epilogue == HK_EPI_SWIGLU) {
@@ -903,6 +1006,7 @@ int hk_gemm_bf16_pair(struct h3_gpu *gpu, const uint16_t *x,
     hk_gemm_args g;
     g.x = x; g.w = w0; g.bias = b0; g.c = c0;
     g.m = m; g.n = n; g.k = k;
+    g.tile_rows = HK_BM;
     g.tiles_m = (m + HK_BM - 1) / HK_BM;
     g.tiles_n = (n + HK_BN - 1) / HK_BN;
     g.x_bytes = (uint32_t)((uint64_t)m * k * 2);
@@ -952,17 +1056,19 @@ static int hk_gemm_bf16_group(struct h3_gpu *gpu, const uint16_t *x,
     memset(&g, 0, sizeof(g));
     g.x = x;
     g.m = m; g.n = n; g.k = k;
-    g.tiles_m = (m + HK_BM - 1) / HK_BM;
+    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
     g.tiles_n = (n + HK_BN - 1) / HK_BN;
+    const uint32_t jb =
+        hk_gemm_row_blocks(m, count * g.tiles_n, k / HK_BK, cus, false);
+    g.tile_rows = 32u * jb;
+    g.tiles_m = (m + g.tile_rows - 1) / g.tile_rows;
     g.x_bytes = (uint32_t)((uint64_t)m * k * 2);
     g.w_bytes = (uint32_t)((uint64_t)n * k * 2);
     g.group_tiles = g.tiles_m * g.tiles_n;
     g.group = table;
     g.tile_count = count * g.group_tiles;
-    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
-    hipLaunchKernelGGL((hk_gemm_mfma<HK_EPI_STORE, true>),
-                       dim3(hk_gemm_grid(g.tile_count, cus)),
-                       dim3(HK_GEMM_THREADS), HK_GEMM_LDS, gpu->stream, g);
+    hk_gemm_launch(gpu, hk_gemm_pick<HK_EPI_STORE, true>(jb), jb,
+                   hk_gemm_grid(g.tile_count, cus), g);
     return 1;
 }
 
