@@ -750,6 +750,71 @@ static void hk_flash_launch(struct h3_gpu *gpu, const hk_attn_args &a,
                            gpu->stream, a);
 }
 
+/* How a dense launch runs: 128- or 256-query workgroups, and the key-range
+ * pieces of the last, sparse round's items (1: whole). */
+struct hk_attn_plan {
+    bool four;
+    uint32_t pieces;
+};
+
+/* Estimated microseconds of `units` items over `tiles` key tiles, in rounds
+ * of `slots`, the last round's items cut into `pieces`: fitted to 324 dense
+ * launches (1-56 heads, 200-9720 rows; 6% rms).  A tile costs less when
+ * fewer items run (clock and caches), and a 128-query item much less while
+ * it has a CU to itself (half the slots); pieces cost a launch and their
+ * partial sums, written and merged. */
+static float hk_attn_estimate(bool four, uint32_t units, uint32_t tiles,
+                              uint32_t slots, uint32_t pieces) {
+    auto tile_us = [&](uint32_t items) {
+        const float fill = (float)items / (float)slots;
+        if (!four) return fill < 1.0f ? 1.43f + 0.29f * fill : 1.85f;
+        return fill <= 0.5f  ? 0.93f + 0.59f * fill
+               : fill < 1.0f ? 1.36f + 0.66f * fill
+                             : 1.93f;
+    };
+    auto rounds = [&](uint32_t items, uint32_t steps) {
+        const uint32_t rest = items % slots;
+        float per = (float)(items / slots) * tile_us(slots);
+        if (rest) per += tile_us(rest);
+        return (four ? 5.2f : 5.1f) + (float)steps * per;
+    };
+    const uint32_t tail = units % slots;
+    if (pieces < 2 || !tail) return rounds(units, tiles);
+    const uint32_t per = (tiles + pieces - 1) / pieces;
+    const uint32_t cut = tail * ((tiles + per - 1) / per);
+    return (units > tail ? rounds(units - tail, tiles) : 0.0f) +
+           rounds(cut, per) + 4.2f + 0.041f * (float)cut;
+}
+
+/* The fastest of 256-query items, whole or with the last round cut into 2-8
+ * pieces, and 128-query items (two a CU, never cut).  Measured at 56 heads
+ * (us, whole 256 / best cut / 128): 300 rows 13.7 / 23.4 / 10.9 (cutting
+ * any sparse round, as this did, cost 24 us there), 1100 rows 58 / 56 / 41
+ * (504 items fit the 512 slots), 1700 rows 97 / 114 / 103, 2378 rows 200 /
+ * 178 / 188, 2700 rows 228 / 220 / 215; at 16 heads 1536 rows take 32 with
+ * 128-query items, 58 cut into 8.  One round that uses over half the
+ * CUs stays whole at 256 queries, where 128 gain nothing (600 rows: 21.3
+ * against 22.5). */
+static hk_attn_plan hk_attn_plan_of(uint32_t q_rows, uint32_t kv_rows,
+                                    uint32_t heads, uint32_t cus) {
+    const uint32_t tiles = (kv_rows + HK_KT - 1) / HK_KT;
+    const uint32_t units = (q_rows + HK_QB - 1) / HK_QB * heads;
+    hk_attn_plan plan = {false, 1};
+    if (units <= cus && units * 2 > cus) return plan;
+    float best = hk_attn_estimate(false, units, tiles, cus, 1);
+    for (uint32_t s = 2; s <= 8 && tiles >= 2 * s; s++) {
+        const float us = hk_attn_estimate(false, units, tiles, cus, s);
+        if (us < best) {
+            best = us;
+            plan.pieces = s;
+        }
+    }
+    const float narrow = hk_attn_estimate(
+        true, (q_rows + 127u) / 128u * heads, tiles, 2 * cus, 1);
+    if (1.02f * narrow < best) return {true, 1};
+    return plan;
+}
+
 int hk_attention_bf16(struct h3_gpu *gpu, const uint16_t *q,
                       const uint16_t *k, const uint16_t *v, uint16_t *o,
                       uint32_t q_rows, uint32_t kv_rows, uint32_t heads,
@@ -827,7 +892,11 @@ int hk_attention_bf16(struct h3_gpu *gpu, const uint16_t *q,
          * workgroup would walk the union of two blocks' lists, and where they
          * differ (the window mask keeps 38 and 27 of 38 tiles in adjacent
          * blocks) half of its waves idle on the other block's tiles. */
-        const bool four = narrow || masked;
+        const uint32_t num_cus =
+            gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
+        const hk_attn_plan plan =
+            hk_attn_plan_of(q_rows, kv_rows, heads, num_cus * HK_WG_PER_CU);
+        const bool four = narrow || masked || plan.four;
         const uint32_t qb_rows = four ? 128u : HK_QB;
         a.q_blocks = (q_rows + qb_rows - 1) / qb_rows;
         a.q_bytes = (uint32_t)q_bytes;
@@ -852,23 +921,26 @@ int hk_attention_bf16(struct h3_gpu *gpu, const uint16_t *q,
         /* With one workgroup per CU the items run in rounds of num_cus.  A
          * sparse last round (the H3 block at 2378 rows: 560 items = 2
          * rounds + 48) is cut along the keys into pieces that fill the
-         * CUs, when that takes at most 0.6 of a round instead of one; a
-         * combine kernel merges the pieces' partial softmax. */
-        const uint32_t cus = (gpu->num_cus > 0 ? (uint32_t)gpu->num_cus
-                                               : 256u) *
-                             (four ? 2u : (uint32_t)HK_WG_PER_CU);
+         * CUs where the plan above finds that faster; a combine kernel
+         * merges the pieces' partial softmax.  Block-sparse items, of
+         * unequal length, are cut when that takes at most 0.6 of a round
+         * instead of one. */
+        const uint32_t cus = num_cus * (four ? 2u : (uint32_t)HK_WG_PER_CU);
         const uint32_t kv_tiles = (kv_rows + HK_KT - 1) / HK_KT;
         const uint32_t tail = units % cus;
-        uint32_t pieces = 1;
-        float best = 1.0f;
-        for (uint32_t s = 2; tail && s <= 8 && kv_tiles >= 2 * s; s++) {
-            const float cost = (float)((tail * s + cus - 1) / cus) / (float)s;
-            if (cost < best - 1e-6f) {
-                best = cost;
-                pieces = s;
+        uint32_t pieces = four || !tail ? 1 : plan.pieces;
+        if (masked) {
+            float best = 1.0f;
+            for (uint32_t s = 2; tail && s <= 8 && kv_tiles >= 2 * s; s++) {
+                const float cost =
+                    (float)((tail * s + cus - 1) / cus) / (float)s;
+                if (cost < best - 1e-6f) {
+                    best = cost;
+                    pieces = s;
+                }
             }
+            if (best > 0.6f) pieces = 1;
         }
-        if (best > 0.6f || narrow) pieces = 1;
         /* scratch: the packed RoPE table, the rotated keys, then the split
          * pieces' partials */
         const size_t table_bytes = ((size_t)a.rope_bytes + 255) & ~(size_t)255;
