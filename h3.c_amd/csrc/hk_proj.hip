@@ -19,109 +19,159 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t hk_proj_rsrc(const void *p,
 /* ------------------------------------------------------------ F32 linear
  *
  * C[M, N] = X[M, K] . W[N, K]^T (+ bias), all F32.  Few rows (the time rows
- * of a schedule), so it is bound by streaming W once; one thread per output
- * walked W with a row stride between lanes and a serial chain of K fmaf.
+ * of a schedule), so it should be bound by streaming W once; one thread per
+ * output walked W with a row stride between lanes and a serial chain of K
+ * fmaf.
  *
- * A workgroup owns 16 columns and up to 16 MB rows, and its eight waves
- * split K: 168 workgroups (the 2688 columns of the time MLP's second layer)
- * then keep 1344 waves loading.  Each lane loads 16 bytes of a W row (and of
- * MB X rows, which L2 serves), DEPTH steps of 16 k ahead of the MFMAs;
- * component j of the four k quarters goes into MFMA j, the same permutation
- * of k on both operands.  The waves' sums meet in LDS in wave order, then
- * the bias is added.  The sum of 8 chains has a smaller rounding error than
- * the single chain had.
+ * A workgroup owns 32 columns, up to 16 MB rows and, where that leaves CUs
+ * idle, one of a few pieces of K (blockIdx.z); its eight waves split the K
+ * range again.  Each lane loads 16 bytes of two W rows and of MB X rows,
+ * DEPTH steps of 32 k ahead of the MFMAs; component j of the four k quarters
+ * goes into MFMA j, the same permutation of k on both operands.  The waves'
+ * sums meet in LDS in wave order; pieces leave partial sums that
+ * hk_linear_f32_reduce adds in piece order, and the bias comes last.  The sum
+ * of many short chains has a smaller rounding error than the single chain
+ * had.
  *
- * Measured (39 rows, 256 -> 5376 and 5376 -> 2688): 10.4 and 41.6 us, from
- * 211 and 2284 us. */
-enum { HK_LF_WAVES = 8 };
+ * X, re-read by every workgroup, is what its rate hangs on: with 16 columns
+ * and all of K per workgroup (168 of them for 5376 -> 2688) 39 rows took 41
+ * us, 10 more for every 16 rows, deeper pipelines or whole-line loads made no
+ * difference; 32 columns and three pieces read half of it, on all CUs.
+ * Measured (39 rows, 256 -> 5376 and 5376 -> 2688, with the reduction):
+ * 8.7 and 27.6 us (22.9 and 4.7), from 211 and 2284. */
+enum { HK_LF_WAVES = 8, HK_LF_BLOCKS = 2 };
+
+struct hk_linear_f32_args {
+    const float *x, *w, *bias;
+    float *c;         /* [M, N], or with pieces their sums [piece][M, N] */
+    uint32_t m, n, k, x_bytes, w_bytes;
+    uint32_t piece_steps; /* 32-wide k steps of a piece */
+};
 
 template <int MB, int DEPTH>
 __global__ void __launch_bounds__(HK_LF_WAVES * 64)
-hk_linear_f32_mfma(const float *x, const float *w, const float *bias,
-                   float *c, uint32_t m, uint32_t n, uint32_t k,
-                   uint32_t x_bytes, uint32_t w_bytes) {
+hk_linear_f32_mfma(hk_linear_f32_args g) {
+    constexpr int NB = HK_LF_BLOCKS;
     extern __shared__ __attribute__((aligned(16))) float hk_lf_red[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r16 = lane & 15u, quad = lane >> 4;
-    const uint32_t n0 = blockIdx.x * 16u, m0 = blockIdx.y * (16u * MB);
-    const __amdgpu_buffer_rsrc_t xr = hk_proj_rsrc(x, x_bytes);
-    const __amdgpu_buffer_rsrc_t wr = hk_proj_rsrc(w, w_bytes);
-    /* this wave's 16-wide k steps */
-    const uint32_t steps = (k + 15u) / 16u;
-    const uint32_t first = steps * wave / HK_LF_WAVES;
-    const uint32_t last = steps * (wave + 1u) / HK_LF_WAVES;
+    const uint32_t n0 = blockIdx.x * (16u * NB);
+    const uint32_t m0 = blockIdx.y * (16u * MB);
+    const uint32_t m = g.m, n = g.n, k = g.k;
+    const __amdgpu_buffer_rsrc_t xr = hk_proj_rsrc(g.x, g.x_bytes);
+    const __amdgpu_buffer_rsrc_t wr = hk_proj_rsrc(g.w, g.w_bytes);
+    /* this wave's 32-wide k steps of the workgroup's piece */
+    const uint32_t begin = blockIdx.z * g.piece_steps;
+    const uint32_t steps = min(g.piece_steps, (k + 31u) / 32u - begin);
+    const uint32_t first = begin + steps * wave / HK_LF_WAVES;
+    const uint32_t last = begin + steps * (wave + 1u) / HK_LF_WAVES;
     /* rows past the end start at the buffer's end and read zeros; so does
      * the part of a last step past K, on both operands */
-    const uint32_t w_off = min(n0 + r16, n) * k * 4u + quad * 16u;
-    uint32_t x_off[MB];
+    uint32_t w_off[NB], x_off[MB];
+#pragma unroll
+    for (int a = 0; a < NB; a++)
+        w_off[a] = min(n0 + 16u * a + r16, n) * k * 4u + quad * 16u;
 #pragma unroll
     for (int b = 0; b < MB; b++)
         x_off[b] = min(m0 + 16u * b + r16, m) * k * 4u + quad * 16u;
-    hk_v4i wf[DEPTH], xf[DEPTH][MB];
+    hk_v4i wf[DEPTH][NB][2], xf[DEPTH][MB][2];
     auto load = [&](int slot, uint32_t step) {
-        const bool in = step < last && step * 16u + quad * 4u < k;
-        wf[slot] = __builtin_amdgcn_raw_buffer_load_b128(
-            wr, in ? w_off + step * 64u : w_bytes, 0, 0);
+        bool in[2];
+#pragma unroll
+        for (uint32_t h = 0; h < 2; h++)
+            in[h] = step < last && step * 32u + h * 16u + quad * 4u < k;
+#pragma unroll
+        for (int a = 0; a < NB; a++)
+#pragma unroll
+            for (uint32_t h = 0; h < 2; h++)
+                wf[slot][a][h] = __builtin_amdgcn_raw_buffer_load_b128(
+                    wr, in[h] ? w_off[a] + step * 128u + h * 64u : g.w_bytes,
+                    0, 0);
 #pragma unroll
         for (int b = 0; b < MB; b++)
-            xf[slot][b] = __builtin_amdgcn_raw_buffer_load_b128(
-                xr, in ? x_off[b] + step * 64u : x_bytes, 0, 0);
+#pragma unroll
+            for (uint32_t h = 0; h < 2; h++)
+                xf[slot][b][h] = __builtin_amdgcn_raw_buffer_load_b128(
+                    xr, in[h] ? x_off[b] + step * 128u + h * 64u : g.x_bytes,
+                    0, 0);
     };
-    hk_f32x4 acc[MB];
+    hk_f32x4 acc[NB][MB];
 #pragma unroll
-    for (int b = 0; b < MB; b++) acc[b] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int a = 0; a < NB; a++)
 #pragma unroll
-    for (int d = 0; d < DEPTH; d++) load(d, first + d);
+        for (int b = 0; b < MB; b++)
+            acc[a][b] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) {
+        load(d, first + d);
+        __builtin_amdgcn_sched_barrier(0); /* in this order: see below */
+    }
     for (uint32_t s = first; s < last; s += DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) {
-            /* steps past the range hold zeros */
-            const hk_f32x4 wv = __builtin_bit_cast(hk_f32x4, wf[d]);
-            hk_f32x4 xv[MB];
+            if (s + d >= last) break;
 #pragma unroll
-            for (int b = 0; b < MB; b++)
-                xv[b] = __builtin_bit_cast(hk_f32x4, xf[d][b]);
+            for (int h = 0; h < 2; h++) {
+                hk_f32x4 wv[NB], xv[MB];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+                for (int a = 0; a < NB; a++)
+                    wv[a] = __builtin_bit_cast(hk_f32x4, wf[d][a][h]);
 #pragma unroll
                 for (int b = 0; b < MB; b++)
-                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        wv[j], xv[b][j], acc[b], 0, 0, 0);
+                    xv[b] = __builtin_bit_cast(hk_f32x4, xf[d][b][h]);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int a = 0; a < NB; a++)
+#pragma unroll
+                        for (int b = 0; b < MB; b++)
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                wv[a][j], xv[b][j], acc[a][b], 0, 0, 0);
+            }
             load(d, s + DEPTH + d);
+            /* keeps the loads here: gathered at the loop's end, they were
+             * all waited for at its top */
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    /* acc[b][i] = C[m0 + 16 b + r16][n0 + 4 quad + i], summed over waves */
+    /* acc[a][b][i] = C[m0 + 16 b + r16][n0 + 16 a + 4 quad + i], summed over
+     * the waves */
     hk_f32x4 *red = (hk_f32x4 *)hk_lf_red;
 #pragma unroll
-    for (int b = 0; b < MB; b++)
-        red[(wave * MB + b) * 64u + lane] = acc[b];
+    for (int a = 0; a < NB; a++)
+#pragma unroll
+        for (int b = 0; b < MB; b++)
+            red[((wave * NB + a) * MB + b) * 64u + lane] = acc[a][b];
     __syncthreads();
-    for (uint32_t t = tid; t < MB * 64u; t += HK_LF_WAVES * 64u) {
+    float *c = g.c + (size_t)blockIdx.z * m * n;
+    for (uint32_t t = tid; t < NB * MB * 64u; t += HK_LF_WAVES * 64u) {
         hk_f32x4 sum = red[t];
 #pragma unroll
-        for (int v = 1; v < HK_LF_WAVES; v++) sum += red[v * MB * 64u + t];
-        const uint32_t row = m0 + (t >> 6) * 16u + (t & 15u);
-        const uint32_t col = n0 + ((t >> 4) & 3u) * 4u;
+        for (int v = 1; v < HK_LF_WAVES; v++)
+            sum += red[v * NB * MB * 64u + t];
+        const uint32_t block = t >> 6;
+        const uint32_t row = m0 + block % MB * 16u + (t & 15u);
+        const uint32_t col =
+            n0 + block / MB * 16u + ((t >> 4) & 3u) * 4u;
         if (row >= m) continue;
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (col + i < n)
                 c[(size_t)row * n + col + i] =
-                    sum[i] + (bias ? bias[col + i] : 0.0f);
+                    sum[i] + (g.bias ? g.bias[col + i] : 0.0f);
     }
 }
 
-template <int MB, int DEPTH>
-static void hk_linear_f32_run(struct h3_gpu *gpu, const float *x,
-                              const float *w, const float *bias, float *c,
-                              uint32_t m, uint32_t n, uint32_t k) {
-    hipLaunchKernelGGL((hk_linear_f32_mfma<MB, DEPTH>),
-                       dim3((n + 15) / 16, (m + 16 * MB - 1) / (16 * MB)),
-                       dim3(HK_LF_WAVES * 64),
-                       HK_LF_WAVES * MB * 64 * sizeof(hk_f32x4), gpu->stream,
-                       x, w, bias, c, m, n, k, (uint32_t)((uint64_t)m * k * 4),
-                       (uint32_t)((uint64_t)n * k * 4));
+/* C = the pieces' sums, in piece order, + bias. */
+__global__ void __launch_bounds__(256)
+hk_linear_f32_reduce(const float *partial, const float *bias, float *c,
+                     uint32_t m, uint32_t n, uint32_t pieces) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= m * n) return;
+    float sum = partial[i];
+    for (uint32_t p = 1; p < pieces; p++) sum += partial[(size_t)p * m * n + i];
+    c[i] = sum + (bias ? bias[i % n] : 0.0f);
 }
 
 bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
@@ -134,14 +184,55 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
         (uint64_t)m * k * 4 + margin >= 0x100000000ull ||
         (uint64_t)n * k * 4 + margin >= 0x100000000ull || m > 65535u * 64u)
         return false;
-    if (m <= 16)
-        hk_linear_f32_run<1, 8>(gpu, x, w, bias, c, m, n, k);
-    else if (m <= 32)
-        hk_linear_f32_run<2, 6>(gpu, x, w, bias, c, m, n, k);
-    else if (m <= 48)
-        hk_linear_f32_run<3, 4>(gpu, x, w, bias, c, m, n, k);
-    else
-        hk_linear_f32_run<4, 4>(gpu, x, w, bias, c, m, n, k);
+    struct {
+        uint32_t blocks;
+        void (*kernel)(hk_linear_f32_args);
+    } const sizes[] = {{1, hk_linear_f32_mfma<1, 4>},
+                       {2, hk_linear_f32_mfma<2, 3>},
+                       {3, hk_linear_f32_mfma<3, 3>},
+                       {4, hk_linear_f32_mfma<4, 2>},
+                       {6, hk_linear_f32_mfma<6, 2>},
+                       {8, hk_linear_f32_mfma<8, 1>}};
+    /* the fewest row blocks of 16 that hold m, at most 8 a workgroup */
+    uint32_t at = 0;
+    while (at < 5 && sizes[at].blocks * 16u < m) at++;
+    const uint32_t mb = sizes[at].blocks;
+    const uint32_t lds =
+        HK_LF_WAVES * HK_LF_BLOCKS * mb * 64 * (uint32_t)sizeof(hk_f32x4);
+    const uint32_t gx = (n + 16 * HK_LF_BLOCKS - 1) / (16 * HK_LF_BLOCKS);
+    const uint32_t gy = (m + 16 * mb - 1) / (16 * mb);
+    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
+    const uint32_t steps = (k + 31u) / 32u;
+    /* pieces of at least 4 steps a wave, while they find idle CUs */
+    uint32_t pieces = gx * gy <= cus ? cus / (gx * gy) : 1u;
+    if (pieces > steps / (4 * HK_LF_WAVES)) pieces = steps / (4 * HK_LF_WAVES);
+    hk_linear_f32_args g = {x, w, bias, c, m, n, k,
+                            (uint32_t)((uint64_t)m * k * 4),
+                            (uint32_t)((uint64_t)n * k * 4), steps};
+    if (pieces > 1) {
+        g.piece_steps = (steps + pieces - 1) / pieces;
+        pieces = (steps + g.piece_steps - 1) / g.piece_steps;
+        float *partial = (float *)hk_splitk_space(
+            gpu, (size_t)pieces * m * n * sizeof(float));
+        if (partial) {
+            g.c = partial;
+            g.bias = NULL;
+        } else { /* no scratch: in one piece */
+            g.piece_steps = steps;
+            pieces = 1;
+        }
+    }
+    if (pieces < 1) pieces = 1;
+    if (lds > 64 * 1024)
+        (void)hipFuncSetAttribute((const void *)sizes[at].kernel,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds);
+    hipLaunchKernelGGL(sizes[at].kernel, dim3(gx, gy, pieces),
+                       dim3(HK_LF_WAVES * 64), lds, gpu->stream, g);
+    if (pieces > 1)
+        hipLaunchKernelGGL(hk_linear_f32_reduce, dim3((m * n + 255) / 256),
+                           dim3(256), 0, gpu->stream, g.c, bias, c, m, n,
+                           pieces);
     return true;
 }
 

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
     (1, 4, 1), (3, 20, 5),          # one step, a step's tail
     (16, 256, 16), (17, 260, 33),   # a full tile, one row and column more
     (33, 128, 47), (48, 96, 64), (49, 2052, 31),
-    (64, 516, 18), (65, 512, 17),   # one and two row blocks
+    (64, 516, 18), (65, 512, 17), (96, 1040, 16), (97, 64, 5),
+    (128, 300, 33), (129, 96, 20),  # every height, one and two row blocks
     (39, 256, 5376), (101, 5376, 2688),
     (5, 7, 9),                      # K % 4 != 0: the general kernel
 ])
