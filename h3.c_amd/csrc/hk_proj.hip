@@ -244,15 +244,16 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
  * through k four at a time, lane quarter q holding k = 4 s + q.
  *
  * Bound by the F32 MFMA rate (1.85 GFLOP for 1792 x 96 -> 5376, 12 us at
- * 157 TFLOP/s; its bytes take 4 us).  A 128-column x 64-row tile per
- * workgroup (four waves of 64 x 32) gives the checkpoint's 5376 columns
- * 42 x 28 workgroups at 1792 rows and 27 KiB of LDS lets four share a CU, so
- * one's loads overlap the others' MFMAs.  LDS holds each row's 32-deep k
- * chunk quarter by quarter (k % 4, then k / 4), so that one 16-byte read
- * feeds four MFMAs; a row pitch of 36 floats spreads 16 rows over all banks.
- * One thread per output had read W rows with a 384-byte stride between
- * lanes: 31.5 us from 493 at 1792 rows, 4.8 from 9.6 at 74 (32 inputs). */
-enum { HK_PL_COLS = 128, HK_PL_ROWS = 64, HK_PL_K = 32, HK_PL_PITCH = 36 };
+ * 155 TFLOP/s; its bytes take 4 us) and a fixed 7 us of starting, filling LDS
+ * and storing.  A 64-column x 64-row tile per workgroup (four waves of
+ * 32 x 32) needs 18 KiB of LDS and 72 registers, so seven share a CU and
+ * one's loads overlap the others' MFMAs; 128 columns (three or four a CU)
+ * took 26.8 us and 7.8 at 192 rows, this 26.1 and 5.4.  LDS holds each row's
+ * 32-deep k chunk quarter by quarter (k % 4, then k / 4), so that one 16-byte
+ * read feeds four MFMAs; a row pitch of 36 floats spreads 16 rows over all
+ * banks.  One thread per output had read W rows with a 384-byte stride
+ * between lanes: 493 us at 1792 rows. */
+enum { HK_PL_COLS = 64, HK_PL_ROWS = 64, HK_PL_K = 32, HK_PL_PITCH = 36 };
 
 __global__ void __launch_bounds__(256)
 hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
@@ -264,22 +265,22 @@ hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t r16 = lane & 15u, quad = lane >> 4;
     const uint32_t n0 = blockIdx.x * HK_PL_COLS, m0 = blockIdx.y * HK_PL_ROWS;
-    const uint32_t wn = (wave >> 1) * 64u, wm = (wave & 1u) * 32u;
+    const uint32_t wn = (wave >> 1) * 32u, wm = (wave & 1u) * 32u;
     /* staging: thread t takes 16-byte piece t % 8 of rows t / 8 + 32 i;
      * rows past the end repeat the last one (their outputs are dropped) */
     const uint32_t piece = tid & 7u, srow = tid >> 3;
-    const float *wp[4], *xp[2];
+    const float *wp[2], *xp[2];
 #pragma unroll
-    for (uint32_t i = 0; i < 4; i++)
+    for (uint32_t i = 0; i < 2; i++)
         wp[i] = w + (size_t)min(n0 + srow + 32u * i, n - 1u) * k + piece * 4u;
 #pragma unroll
     for (uint32_t i = 0; i < 2; i++)
         xp[i] = x + (size_t)min(m0 + srow + 32u * i, m - 1u) * k + piece * 4u;
-    hk_f32x4 wv[4], xv[2];
+    hk_f32x4 wv[2], xv[2];
     auto load = [&](uint32_t k0) {
         if (k0 + piece * 4u >= k) return;
 #pragma unroll
-        for (int i = 0; i < 4; i++) wv[i] = *(const hk_f32x4 *)(wp[i] + k0);
+        for (int i = 0; i < 2; i++) wv[i] = *(const hk_f32x4 *)(wp[i] + k0);
 #pragma unroll
         for (int i = 0; i < 2; i++) xv[i] = *(const hk_f32x4 *)(xp[i] + k0);
     };
@@ -287,22 +288,21 @@ hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
 #pragma unroll
         for (int e = 0; e < 4; e++) base[e * 8 + piece] = v[e];
     };
-    hk_f32x4 acc[4][2];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t col = n0 + wn + 16u * a + quad * 4u + i;
-            const float b = bias && col < n ? bias[col] : 0.0f;
-            acc[a][0][i] = acc[a][1][i] = b;
-        }
-#pragma unroll
-    for (int i = 0; i < 4; i++) wv[i] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 2; i++) wv[i] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     xv[0] = xv[1] = wv[0];
     load(0);
+    hk_f32x4 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const uint32_t col = n0 + wn + 16u * a + quad * 4u;
+        acc[a][0] = bias && col < n ? *(const hk_f32x4 *)(bias + col)
+                                    : hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        acc[a][1] = acc[a][0];
+    }
     for (uint32_t k0 = 0; k0 < k; k0 += HK_PL_K) {
 #pragma unroll
-        for (uint32_t i = 0; i < 4; i++)
+        for (uint32_t i = 0; i < 2; i++)
             put(lds + (srow + 32u * i) * HK_PL_PITCH, wv[i]);
 #pragma unroll
         for (uint32_t i = 0; i < 2; i++)
@@ -312,9 +312,9 @@ hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
         const uint32_t steps = min((k - k0) / 4u, 8u);
 #pragma unroll
         for (uint32_t g = 0; g < 2; g++) {
-            hk_f32x4 wf[4], xf[2];
+            hk_f32x4 wf[2], xf[2];
 #pragma unroll
-            for (int a = 0; a < 4; a++)
+            for (int a = 0; a < 2; a++)
                 wf[a] = *(const hk_f32x4 *)(
                     lds + (wn + 16u * a + r16) * HK_PL_PITCH + quad * 8u +
                     g * 4u);
@@ -327,7 +327,7 @@ hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
             for (uint32_t s = 0; s < 4; s++)
                 if (g * 4u + s < steps)
 #pragma unroll
-                    for (int a = 0; a < 4; a++)
+                    for (int a = 0; a < 2; a++)
 #pragma unroll
                         for (int b = 0; b < 2; b++)
                             acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(
@@ -341,7 +341,7 @@ hk_patch_linear_mfma(const float *x, const float *w, const float *bias,
         if (row >= m) continue;
         uint16_t *dst = out + (size_t)(row_map ? row_map[row] : row) * n;
 #pragma unroll
-        for (int a = 0; a < 4; a++) {
+        for (int a = 0; a < 2; a++) {
             const uint32_t col = n0 + wn + 16u * a + quad * 4u;
             if (col < n)
                 *(uint2 *)(dst + col) =
@@ -356,7 +356,8 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
                      const uint32_t *row_map, uint32_t m, uint32_t n,
                      uint32_t k) {
     if (!k || k % 4 || n % 4 || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
-        ((uintptr_t)out & 7) || m > 65535u * HK_PL_ROWS)
+        ((uintptr_t)bias & 15) || ((uintptr_t)out & 7) ||
+        m > 65535u * HK_PL_ROWS)
         return false;
     hipLaunchKernelGGL(hk_patch_linear_mfma,
                        dim3((n + HK_PL_COLS - 1) / HK_PL_COLS,
