@@ -385,7 +385,9 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
  * a workgroup with NB = 3 (half of it weights).  Loading x, norm, shift and
  * scale as MFMA fragments instead (16 lanes repeating each modulation piece)
  * took 41-44 us at 1792 rows x 96 outputs and 21 us at 74 rows x 32; this
- * takes 28.7 and 16.7 us.  One workgroup per row: 563 and 198. */
+ * takes 24.2 and 15.4 us, with the modulation rows' numbers, the modulation
+ * and a half's first weights loaded ahead of their use (28.7 and 16.7
+ * without).  One workgroup per row: 563 and 198. */
 enum { HK_HEAD_WAVES = 16 };
 
 struct hk_head_args {
@@ -410,7 +412,7 @@ hk_adaln_head_mfma(hk_head_args a) {
     __shared__ float squares[HK_HEAD_WAVES][ROWS];
     __shared__ float inverses[ROWS];
     /* weight steps in flight: as many as the registers hold */
-    constexpr uint32_t AHEAD = NB * ROWS > 32 ? 2 : 3;
+    constexpr uint32_t AHEAD = NB > 3 ? 1 : NB * ROWS > 32 ? 2 : 3;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r16 = lane & 15u, quad = lane >> 4;
@@ -422,11 +424,43 @@ hk_adaln_head_mfma(hk_head_args a) {
     const bool mine = col < a.width;
     /* rows past the end repeat the last one; their outputs are dropped */
     auto row_of = [&](uint32_t r) { return min(row0 + r, a.rows - 1u); };
+    /* weight rows past N repeat the last one; those columns are dropped */
+    const uint16_t *wr[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        wr[b] = a.w + (size_t)min(n0 + 16u * b + r16, a.n - 1u) * a.width +
+                quad * 8u;
+    /* AHEAD steps' weights in flight, a half's first ones from before its
+     * rows are ready; steps past the half repeat its last one */
+    hk_bf16x8 wf[AHEAD][NB];
+    auto load = [&](uint32_t first, uint32_t count, uint32_t s0) {
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++)
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+                wf[u][b] = *(const hk_bf16x8 *)(
+                    wr[b] +
+                    (first + min(s0 + u * HK_HEAD_WAVES, count - 1u)) * 32u);
+    };
+    if (ROWS == 4) load(0, half_steps, wave); /* the registers allow it */
     const uint32_t at = min(col, a.width - 8u); /* loads without a branch */
+    /* every row's modulation row, one a lane: loaded row by row, they were
+     * a chain of ROWS loads */
+    const uint32_t maps = a.row_map[row_of(lane % ROWS)];
     uint4 xv[ROWS];
 #pragma unroll
     for (uint32_t r = 0; r < ROWS; r++)
         xv[r] = *(const uint4 *)(a.x + (size_t)row_of(r) * a.width + at);
+    const uint4 nw = *(const uint4 *)(a.norm + at);
+    uint4 sh, sc;
+    auto load_mod = [&](uint32_t map) {
+        const uint16_t *mod = a.mod + (size_t)map * a.slots * a.width + at;
+        sh = *(const uint4 *)(mod + (size_t)a.shift_slot * a.width);
+        sc = *(const uint4 *)(mod + (size_t)a.scale_slot * a.width);
+    };
+    /* readlane: a branch on the map must not become a lane mask */
+    uint32_t map = __builtin_amdgcn_readlane(maps, 0);
+    load_mod(map);
     /* ROWS sums over the wave's 64 lanes: each exchange halves the rows a
      * lane carries, so that the lane's top bits end up naming the row; the
      * other bits are summed as usual */
@@ -470,21 +504,10 @@ hk_adaln_head_mfma(hk_head_args a) {
         if (blockIdx.y == 0 && row0 + tid < a.rows)
             a.inverse[row0 + tid] = inverse;
     }
-    const uint4 nw = *(const uint4 *)(a.norm + at);
-    uint4 sh, sc;
-    auto load_mod = [&](uint32_t map) {
-        const uint16_t *mod = a.mod + (size_t)map * a.slots * a.width + at;
-        sh = *(const uint4 *)(mod + (size_t)a.shift_slot * a.width);
-        sc = *(const uint4 *)(mod + (size_t)a.scale_slot * a.width);
-    };
-    /* readfirstlane: a branch on the map must not become a lane mask */
-    uint32_t map = __builtin_amdgcn_readfirstlane(a.row_map[row_of(0)]);
-    load_mod(map);
     __syncthreads();
 #pragma unroll
     for (uint32_t r = 0; r < ROWS; r++) {
-        const uint32_t next =
-            __builtin_amdgcn_readfirstlane(a.row_map[row_of(r)]);
+        const uint32_t next = __builtin_amdgcn_readlane(maps, r);
         if (next != map) {
             map = next;
             load_mod(map);
@@ -507,15 +530,10 @@ hk_adaln_head_mfma(hk_head_args a) {
         asm volatile("" : "+v"(xv[r].x), "+v"(xv[r].y), "+v"(xv[r].z),
                           "+v"(xv[r].w));
     }
-    /* weight rows past N repeat the last one; those columns are dropped */
-    const uint16_t *wr[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-        wr[b] = a.w + (size_t)min(n0 + 16u * b + r16, a.n - 1u) * a.width +
-                quad * 8u;
     hk_f32x4 acc[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) acc[b] = hk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (ROWS != 4) load(0, half_steps, wave);
 #pragma unroll
     for (uint32_t h = 0; h < 2; h++) {
         const uint32_t first = h * half_steps;
@@ -527,20 +545,6 @@ hk_adaln_head_mfma(hk_head_args a) {
             for (uint32_t r = 0; r < ROWS; r++)
                 *(uint4 *)(dst + r * pitch) = xv[r];
         }
-        /* AHEAD steps' weights in flight, the first ones across the
-         * barrier; steps past the half repeat its last one */
-        hk_bf16x8 wf[AHEAD][NB];
-        auto load = [&](uint32_t s0) {
-#pragma unroll
-            for (uint32_t u = 0; u < AHEAD; u++)
-#pragma unroll
-                for (int b = 0; b < NB; b++)
-                    wf[u][b] = *(const hk_bf16x8 *)(
-                        wr[b] +
-                        (first + min(s0 + u * HK_HEAD_WAVES, count - 1u)) *
-                            32u);
-        };
-        if (wave < count) load(wave);
         __syncthreads();
         for (uint32_t s0 = wave; s0 < count; s0 += AHEAD * HK_HEAD_WAVES) {
 #pragma unroll
@@ -556,8 +560,10 @@ hk_adaln_head_mfma(hk_head_args a) {
                         wf[u][b], xf, acc[b], 0, 0, 0);
             }
             if (s0 + AHEAD * HK_HEAD_WAVES < count)
-                load(s0 + AHEAD * HK_HEAD_WAVES);
+                load(first, count, s0 + AHEAD * HK_HEAD_WAVES);
         }
+        if (!h && steps > half_steps)
+            load(half_steps, steps - half_steps, wave);
     }
     __syncthreads();
     /* acc[b][i] = out[row0 + r16][n0 + 16 b + 4 quad + i], summed over the
@@ -584,9 +590,17 @@ static void hk_head_run(struct h3_gpu *gpu, const hk_head_args &a) {
     const size_t tile = (size_t)ROWS * hk_head_pitch(a.width);
     const size_t sums = (size_t)HK_HEAD_WAVES * NB * 64 * sizeof(hk_f32x4);
     const size_t lds = tile > sums ? tile : sums;
-    (void)hipFuncSetAttribute((const void *)hk_adaln_head_mfma<NB, ROWS>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)lds);
+    /* over 64 KiB, the kernel's limit is raised (each process and device
+     * once to the most that a width can need) */
+    static uint64_t ready = 0;
+    const uint64_t bit = 1ull << (gpu->device & 63);
+    if (lds > 64 * 1024 && !(ready & bit)) {
+        (void)hipFuncSetAttribute(
+            (const void *)hk_adaln_head_mfma<NB, ROWS>,
+            hipFuncAttributeMaxDynamicSharedMemorySize,
+            (int)((size_t)ROWS * hk_head_pitch(HK_HEAD_WAVES * 64 * 8)));
+        ready |= bit;
+    }
     hipLaunchKernelGGL((hk_adaln_head_mfma<NB, ROWS>),
                        dim3((a.rows + ROWS - 1) / ROWS,
                             (a.n + 16 * NB - 1) / (16 * NB)),
@@ -607,15 +621,17 @@ bool hk_adaln_head(struct h3_gpu *gpu, const uint16_t *x, float *inverse,
     const hk_head_args a = {x,       norm, mod, w,     bias,  row_map,
                             inverse, out,  rows, width, n,    slots,
                             shift_slot, scale_slot, epsilon};
-    /* 4 rows a workgroup while one round of workgroups covers them (16.7 us
-     * against 22.0 with 16 at 74 rows x 32, where a workgroup's own chain of
+    /* 4 rows a workgroup while one round of workgroups covers them (15.4 us
+     * against 22 with 16 at 74 rows x 32, where a workgroup's own chain of
      * steps is all that counts), else 16, which read the weights a quarter
-     * as often */
+     * as often; 96 columns a workgroup where 48 would need a second round
+     * (2835 rows: 40.4 us against 50.7), else 48 (1792: 24.2) */
+    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
     const uint32_t groups = n <= 32 ? 1u : (n + 47u) / 48u;
-    const bool few = (rows + 3u) / 4u * groups <= (uint32_t)gpu->num_cus;
-    if (n <= 32 && few) hk_head_run<2, 4>(gpu, a);
+    if (n <= 32 && (rows + 3u) / 4u <= cus) hk_head_run<2, 4>(gpu, a);
     else if (n <= 32) hk_head_run<2, 16>(gpu, a);
-    else if (few) hk_head_run<3, 4>(gpu, a);
-    else hk_head_run<3, 16>(gpu, a);
+    else if ((rows + 3u) / 4u * groups <= cus) hk_head_run<3, 4>(gpu, a);
+    else if ((rows + 15u) / 16u * groups <= cus) hk_head_run<3, 16>(gpu, a);
+    else hk_head_run<6, 16>(gpu, a);
     return true;
 }
