@@ -309,23 +309,31 @@ extern "C" int h3_hip_gemm_trace_read(uint64_t *out, size_t entries) {
  * offset; rows past M or N keep a lane offset beyond the buffer and read
  * zeros.
  *
+ * W's loads are marked non-temporal: read once, W would push X and the sums
+ * out of L2 (39 rows x 2688 -> 96768: 84 us against 97, 6.2 TB/s; 8 x 14336
+ * -> 5376: 28.6 against 32.4; 120 x 5376 -> 21504: 68 against 73).  Loading
+ * W as 16x16x32 fragments without the LDS turn took 85 for that last one.
+ *
  * XA = 3 hides X's L2 latency behind two steps: with one stage ahead every
  * step waited for it where a CU has only one or two workgroups (40 rows x
- * 5376 -> 21504, 168 workgroups: 48.4 us against 56; 120 rows: 65 against
- * 94).  With three rounds of workgroups and 64 rows or fewer, XA = 1 is
- * 3-4% ahead (39 rows x 2688 -> 96768: 96.6 us against 100): its smaller
- * LDS lets more workgroups share a CU.
+ * 5376 -> 21504, 168 workgroups: 46.7 us against 52.8).  With three rounds of
+ * workgroups and 33 to 64 rows, XA = 1 is 1.5% ahead (39 rows x 2688 ->
+ * 96768: 89.1 us against 90.5 in one run): its smaller LDS lets more
+ * workgroups share a CU.
  *
  * Where one workgroup per 128 columns leaves CUs idle, K is split into as
  * many pieces as there are CUs for (blockIdx.y), which write F32 sums that
- * hk_skinny_reduce adds: 8 x 14336 -> 5376 takes 32 us instead of 146, 120
- * rows 45 instead of 231.  Two workgroups a CU were slower on all but one
+ * hk_skinny_reduce adds: 8 x 14336 -> 5376 takes 28.6 us instead of 146, 120
+ * rows 41 instead of 231.  Two workgroups a CU were slower on all but one
  * shape (34 us, 45-53 us): each piece pays its own start and its sums.
  *
  * Ordering: a step waits until X(s) has landed (loads retire in order; W(s)
  * is a register result the compiler waits for), synchronises, stages
  * X(s + XA) into the buffer every wave finished reading in step s - 1, issues
  * W(s + 3) and computes. */
+/* the non-temporal (streaming) cache policy of a buffer load */
+enum { HK_LOAD_ONCE = 2 };
+
 struct hk_skinny_args {
     const uint16_t *x, *w, *bias;
     uint16_t *c;
@@ -393,7 +401,8 @@ hk_gemm_skinny(hk_skinny_args g) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
             wf[slot][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                wr, wo[q] | dead(step), (base + step) * 128u, 0);
+                wr, wo[q] | dead(step), (base + step) * 128u,
+                HK_LOAD_ONCE);
     };
     /* fragment of X rows mb*32 + row, logical chunk 2q + half */
     auto read_x = [&](int buf, int mb, int q) {
