@@ -860,7 +860,7 @@ static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
     if (splits > 1) {
         g.partial = scratch ? scratch
                             : (float *)hk_splitk_space(gpu, bytes);
-        if (!g.partial) return 0;
+        if (!g.partial) splits = 1; /* no scratch: in one piece */
     }
     const dim3 grid(wgs, splits > 1 ? splits : 1u, problems);
     /* several rounds of few rows: one X stage ahead (both timed above) */

@@ -213,9 +213,9 @@ int h3_hip_head_rms_norm_group_bf16(h3_gpu *gpu, const h3_gpu_tensor *table,
 /* Two projections of one input, output0 = X . weight0^T + bias0 and
  * output1 = X . weight1^T + bias1, each exactly as h3_gpu_linear_bf16
  * computes it (f32 accumulation, one bf16 rounding).  Small launches
- * (together at most half the CUs' worth of 256x256 tiles, such as the
- * text's cross-attention K and V) share one split-K launch; others run as
- * two linears.  Biases may be NULL.  No reference counterpart: the
+ * (over 128 rows and together at most half the CUs' worth of 256x256 tiles,
+ * such as the text's cross-attention K and V) share one split-K launch;
+ * others run as two linears.  Biases may be NULL.  No reference counterpart: the
  * reference has no cross-attention. */
 int h3_hip_linear_pair_bf16(h3_gpu *gpu, h3_gpu_tensor *output0,
                             h3_gpu_tensor *output1,
@@ -227,8 +227,8 @@ int h3_hip_linear_pair_bf16(h3_gpu *gpu, h3_gpu_tensor *output0,
                             uint32_t input_dim, uint32_t output_dim);
 
 /* h3_gpu_linear_bf16 that allocates nothing: the same kernels and the same
- * results, with the split-K partial tiles (used when the last round of
- * 256x256 tiles would leave over half the CUs idle) in a static 64 MiB
+ * results, with the split-K partial sums (used when the last round of tiles,
+ * or a launch of at most 128 rows, would leave CUs idle) in a static 64 MiB
  * device array per GPU instead of the context's on-demand scratch.  A
  * launch whose split would need more fails with an error naming the size.
  * The array (256 CUs x one 256x256 f32 tile) is resident on every GPU the
