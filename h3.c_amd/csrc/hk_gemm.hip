@@ -47,6 +47,7 @@
  */
 #include "hk_common.h"
 #include "hk_internal.h"
+#include "hk_skinny.h"
 
 #include <pthread.h>
 #include <string.h>
@@ -69,8 +70,6 @@
 #define HK_GROUP_M 8
 /* rows the skinny GEMM takes: four 32-row MFMA blocks */
 #define HK_SKINNY_ROWS 128u
-/* its operands' bytes stay below this bit, which marks a dead offset */
-#define HK_SKINNY_LIMIT 0x80000000u
 
 typedef int hk_v4i __attribute__((ext_vector_type(4)));
 typedef int hk_v2i __attribute__((ext_vector_type(2)));
@@ -361,7 +360,7 @@ hk_gemm_skinny(hk_skinny_args g) {
     const uint32_t base = g.partial ? blockIdx.y * g.split_steps : 0u;
     const uint32_t steps =
         g.partial ? min(g.split_steps, k / 64u - base) : k / 64u;
-    constexpr int D = 4;
+    constexpr int D = HK_SKINNY_RING;
     constexpr uint32_t XSTAGE = MB * 32u * 128u; /* bytes of X per k step */
     /* XA + 1 X stages, then the four waves' 4-KiB W buffers */
     extern __shared__ __attribute__((aligned(16))) uint8_t hk_xs[];
@@ -387,22 +386,20 @@ hk_gemm_skinny(hk_skinny_args g) {
         const uint32_t chunk = (p & 7u) ^ hk_swz_key(r);
         xo[i] = (min(r, m) * k + chunk * 8u) * 2u;
     }
-    auto dead = [&](uint32_t step) {
-        return step < steps ? 0u : HK_SKINNY_LIMIT;
-    };
     auto stage_x = [&](int buf, uint32_t step) {
 #pragma unroll
         for (int i = 0; i < MB; i++)
             hk_dma16(xr, hk_xs + buf * XSTAGE + (256u * i + wave * 64u) * 16u,
-                     xo[i] | dead(step), (base + step) * 128u);
+                     xo[i] | hk_skinny_dead(step, steps),
+                     hk_skinny_k_bytes(base + step, k / 64u));
     };
     hk_v4i wf[D][4];
     auto load_w = [&](int slot, uint32_t step) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
             wf[slot][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                wr, wo[q] | dead(step), (base + step) * 128u,
-                HK_LOAD_ONCE);
+                wr, wo[q] | hk_skinny_dead(step, steps),
+                hk_skinny_k_bytes(base + step, k / 64u), HK_LOAD_ONCE);
     };
     /* fragment of X rows mb*32 + row, logical chunk 2q + half */
     auto read_x = [&](int buf, int mb, int q) {
@@ -416,9 +413,9 @@ hk_gemm_skinny(hk_skinny_args g) {
     for (int mb = 0; mb < MB; mb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[mb][r] = 0.0f;
-    /* Steps past the end load zeros (offsets beyond the buffers, no memory
-     * touched) and add nothing, so the loop has no branch: behind one, the
-     * compiler drains every load in flight. */
+    /* Steps past the end load zeros (lane offsets beyond the buffers, no
+     * memory touched) and add nothing, so the loop has no branch: behind one,
+     * the compiler drains every load in flight. */
 #pragma unroll
     for (uint32_t d = 0; d + 1 < D; d++) {
         if (d < XA) stage_x(d, d);
