@@ -413,13 +413,20 @@ hk_gemm_skinny(hk_skinny_args g) {
     for (int mb = 0; mb < MB; mb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[mb][r] = 0.0f;
+    /* The waits below count loads: a step's X loads must leave before its W
+     * loads, and steps in order.  Nothing else orders them (they write LDS
+     * and registers) up to the next step's barrier, which they do not
+     * cross. */
+    auto in_order = [] { __builtin_amdgcn_sched_barrier(0); };
     /* Steps past the end load zeros (lane offsets beyond the buffers, no
      * memory touched) and add nothing, so the loop has no branch: behind one,
      * the compiler drains every load in flight. */
 #pragma unroll
     for (uint32_t d = 0; d + 1 < D; d++) {
         if (d < XA) stage_x(d, d);
+        in_order();
         load_w(d, d);
+        in_order();
     }
     for (uint32_t s0 = 0; s0 < steps; s0 += D) {
 #pragma unroll
@@ -435,6 +442,7 @@ hk_gemm_skinny(hk_skinny_args g) {
              * steps ahead included */
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             stage_x((d + XA) % (XA + 1), s + XA);
+            in_order();
             load_w((d + 3) % D, s + 3);
             /* W(s)'s lines into the wave's buffer and back out as
              * fragments (a wave's LDS operations run in order: no

@@ -15,6 +15,7 @@ csrc/hk_gemm.hip as the Makefile does
 first and the last MFMA of every kernel instance, and requires none of
 those.  It needs hipcc, not a GPU.
 """
+import functools
 import os
 import re
 import shutil
@@ -40,7 +41,9 @@ INSTANCES = {
 BAD = re.compile(r"\b(v_accvgpr_mov_b32|v_accvgpr_write_b32|scratch_\w+)\b")
 
 
-def _k_loop_offenders(extra):
+@functools.lru_cache(maxsize=None)
+def _assembly(*extra):
+    """The lines of csrc/hk_gemm.hip's device assembly."""
     work = tempfile.mkdtemp(prefix="hk_isa_")
     try:
         subprocess.run([HIPCC, *FLAGS, *extra, "--save-temps", "-c", SRC,
@@ -49,15 +52,23 @@ def _k_loop_offenders(extra):
         asm = [f for f in os.listdir(work)
                if f.endswith(".s") and "amdgcn" in f]
         assert asm, "no device assembly written"
-        text = open(os.path.join(work, asm[0])).read().splitlines()
+        return open(os.path.join(work, asm[0])).read().splitlines()
     finally:
         shutil.rmtree(work, ignore_errors=True)
+
+
+def _body(text, sym):
+    start = text.index(next(l for l in text if l.startswith(sym + ":")))
+    end = next(i for i in range(start + 1, len(text))
+               if text[i].startswith(".Lfunc_end"))
+    return text[start:end]
+
+
+def _k_loop_offenders(extra):
+    text = _assembly(*extra)
     found = {}
     for name, sym in INSTANCES.items():
-        start = text.index(next(l for l in text if l.startswith(sym + ":")))
-        end = next(i for i in range(start + 1, len(text))
-                   if text[i].startswith(".Lfunc_end"))
-        body = text[start:end]
+        body = _body(text, sym)
         mfma = [i for i, l in enumerate(body) if "v_mfma_" in l]
         assert len(mfma) == 128, (name, len(mfma))
         loop = body[mfma[0]:mfma[-1]]
@@ -85,3 +96,27 @@ def test_gemm_k_loop_has_no_accumulator_copies_or_scratch(extra):
     offenders = _k_loop_offenders(extra)
     bad = {k: (len(v), v[:3]) for k, v in offenders.items() if v}
     assert not bad, bad
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+@pytest.mark.parametrize("mb,ahead", [(1, 1), (1, 3), (2, 1), (2, 3), (3, 3),
+                                      (4, 3)])
+def test_skinny_loads_leave_in_the_order_its_waits_count(mb, ahead):
+    """hk_gemm_skinny<MB, XA> waits until all but the last 4 + (XA - 1)(MB + 4)
+    loads have landed, which is X of the step at hand only if every step's MB
+    X loads (to LDS) leave before its four W loads, and steps in order."""
+    body = _body(_assembly(),
+                 f"_Z14hk_gemm_skinnyILi{mb}ELi{ahead}EEv14hk_skinny_args")
+    loads = "".join("X" if re.search(r"\blds\b", l) else "W"
+                    for l in body if "buffer_load_" in l)
+    step = "X" * mb + "WWWW"
+    ring = "".join("X" * mb * (d < ahead) + "WWWW" for d in range(3))
+    assert loads == ring + 4 * step
+    mfma = [i for i, l in enumerate(body) if "v_mfma_" in l]
+    assert len(mfma) == 4 * 4 * mb
+    loop = body[mfma[0]:mfma[-1]]
+    assert not [l for l in loop if "s_cbranch" in l or "scratch_" in l]
+    # the kernel's own waits, apart from the compiler's
+    asm = re.findall(r"#ASMSTART\n\s*s_waitcnt vmcnt\((\d+)\)",
+                     "\n".join(body))
+    assert asm == [str(4 + (ahead - 1) * (mb + 4))] * 4
