@@ -590,11 +590,13 @@ static void hk_head_run(struct h3_gpu *gpu, const hk_head_args &a) {
     const size_t tile = (size_t)ROWS * hk_head_pitch(a.width);
     const size_t sums = (size_t)HK_HEAD_WAVES * NB * 64 * sizeof(hk_f32x4);
     const size_t lds = tile > sums ? tile : sums;
-    /* over 64 KiB, the kernel's limit is raised (each process and device
-     * once to the most that a width can need) */
+    /* over 64 KiB with its static LDS (squares and inverses), the kernel's
+     * limit is raised (each process and device once, to the most that a
+     * width can need) */
+    const size_t fixed = (HK_HEAD_WAVES + 1) * ROWS * sizeof(float);
     static uint64_t ready = 0;
     const uint64_t bit = 1ull << (gpu->device & 63);
-    if (lds > 64 * 1024 && !(ready & bit)) {
+    if (lds + fixed > 64 * 1024 && !(ready & bit)) {
         (void)hipFuncSetAttribute(
             (const void *)hk_adaln_head_mfma<NB, ROWS>,
             hipFuncAttributeMaxDynamicSharedMemorySize,

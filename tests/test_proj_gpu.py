@@ -97,6 +97,7 @@ def test_patch_linear_tiles_bit_exact(gpu, rows, k, n, mapped):
     (33, 5376, 32), (3, 512, 97), (2, 8192, 48),
     (1025, 64, 32), (517, 96, 33),  # 16 rows a workgroup
     (2049, 64, 96), (2100, 5376, 50),  # and 96 columns
+    (1025, 4032, 32), (1040, 4000, 96),  # just over 64 KiB of LDS
     (4, 8224, 96), (4, 264, 8),  # the general kernel
 ])
 @pytest.mark.parametrize("shared", [True, False])

@@ -1,0 +1,27 @@
+"""Which kernels a call launches, on 256 CUs, without a GPU (launches.py)."""
+import pytest
+
+from launches import calls_made
+
+
+def head(rows, width, n):
+    return ["h3_gpu_adaln_linear_bf16", ["bf16", rows * n], ["f32", rows],
+            ["bf16", rows * width], 0, ["bf16", width], ["bf16", 2 * width],
+            ["u32", rows], ["bf16", n * width], ["bf16", n], rows, width, n,
+            2, 0, 1, 1e-5]
+
+
+@pytest.mark.parametrize("rows,n", [(1040, 32), (1040, 96), (2100, 96)])
+@pytest.mark.parametrize("width", [3968, 4000, 4032, 4064, 5376, 8192])
+def test_head_lds_limit(rows, n, width):
+    """Dynamic LDS plus the kernel's static 16 + 1 floats a row stay within
+    64 KiB, or the kernel's limit is raised first; a fresh process each, since
+    a limit once raised stays."""
+    (ok, error, (launch,)), = calls_made([head(rows, width, n)])
+    assert ok, error
+    assert launch.kernel.startswith("hk_adaln_head_mfma<")
+    block_rows = int(launch.kernel.split(", ")[1].rstrip(">"))
+    assert block_rows == 16
+    assert launch.lds <= launch.lds_limit
+    if launch.lds + 17 * 4 * block_rows > 64 * 1024:
+        assert launch.lds_limit > 64 * 1024
