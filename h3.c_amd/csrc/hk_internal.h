@@ -53,8 +53,9 @@ struct h3_gpu {
     size_t workspace_bytes;
     void *splitk; /* f32 partial tiles of split-K GEMMs */
     size_t splitk_bytes;
-    /* H3_HIP_REFERENCE=1: route GEMM and attention through the simple
-     * (sequential-k / two-pass) reference kernels */
+    /* H3_HIP_REFERENCE=1: route GEMM, attention and the small projections
+     * through the simple (sequential-k / two-pass / one thread or workgroup
+     * an output or row) kernels */
     int reference_kernels;
     /* per-op event timing */
     struct hk_timing *timing;
@@ -175,7 +176,8 @@ int hk_attention_reference(struct h3_gpu *gpu, const uint16_t *q,
                            uint32_t head_dim, float scale, int head_major);
 
 /* C[M,N] = X[M,K] . W[N,K]^T (+ bias) in F32 on the matrix cores; false (and
- * nothing launched) for a shape or alignment it does not take. */
+ * nothing launched) for a shape or alignment it does not take, and under
+ * H3_HIP_REFERENCE=1. */
 bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
                    const float *bias, float *c, uint32_t m, uint32_t n,
                    uint32_t k);

@@ -180,8 +180,8 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
     /* 16-byte loads; offsets up to a step past the end of a row past the
      * end stay below 2^32 */
     const uint64_t margin = 4ull * k + 4096;
-    if (!k || k % 4 || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
-        (uint64_t)m * k * 4 + margin >= 0x100000000ull ||
+    if (gpu->reference_kernels || !k || k % 4 || ((uintptr_t)x & 15) ||
+        ((uintptr_t)w & 15) || (uint64_t)m * k * 4 + margin >= 0x100000000ull ||
         (uint64_t)n * k * 4 + margin >= 0x100000000ull || m > 65535u * 64u)
         return false;
     struct {
@@ -355,9 +355,9 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
                      const float *bias, uint16_t *out,
                      const uint32_t *row_map, uint32_t m, uint32_t n,
                      uint32_t k) {
-    if (!k || k % 4 || n % 4 || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
-        ((uintptr_t)bias & 15) || ((uintptr_t)out & 7) ||
-        m > 65535u * HK_PL_ROWS)
+    if (gpu->reference_kernels || !k || k % 4 || n % 4 ||
+        ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
+        ((uintptr_t)bias & 15) || ((uintptr_t)out & 7) || m > 65535u * HK_PL_ROWS)
         return false;
     hipLaunchKernelGGL(hk_patch_linear_mfma,
                        dim3((n + HK_PL_COLS - 1) / HK_PL_COLS,
@@ -616,8 +616,8 @@ bool hk_adaln_head(struct h3_gpu *gpu, const uint16_t *x, float *inverse,
                    uint32_t width, uint32_t n, uint32_t slots,
                    uint32_t shift_slot, uint32_t scale_slot, float epsilon) {
     /* a thread per 8 columns, loaded 16 bytes at a time */
-    if (width % 32 || width > HK_HEAD_WAVES * 64 * 8 || !n ||
-        n > 65535u * 32u || ((uintptr_t)x & 15) || ((uintptr_t)norm & 15) ||
+    if (gpu->reference_kernels || width % 32 ||
+        width > HK_HEAD_WAVES * 64 * 8 || !n || n > 65535u * 32u || ((uintptr_t)x & 15) || ((uintptr_t)norm & 15) ||
         ((uintptr_t)mod & 15) || ((uintptr_t)w & 15))
         return false;
     const hk_head_args a = {x,       norm, mod, w,     bias,  row_map,

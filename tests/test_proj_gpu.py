@@ -4,6 +4,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import h3hip
 import oracle
 from conftest import assert_close, rand_bf16, to_f32
 
@@ -124,3 +125,42 @@ def test_adaln_head_tiles(gpu, rows, width, n, shared):
                 slots, 2, 0, C.c_float(1e-5))
         np.testing.assert_allclose(gpu.read_f32(tinv), inv, rtol=1e-5)
         assert_close(gpu.read_bf16(out), want, what="head", chained=1)
+
+
+def test_simple_kernels_agree(gpu, monkeypatch):
+    """The three projections at the models' widths against the simple kernels
+    of H3_HIP_REFERENCE=1: F32 sums within both orders' bounds (each K + 16
+    half-ulps of the sum of magnitudes), the patch projection bit for bit, the
+    head within the composite bound."""
+    rng = np.random.default_rng(5)
+    f32 = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    m, k, n = 39, 5376, 2688
+    x, w, b = f32(m, k), f32(n, k) * np.float32(0.02), f32(n)
+    px, pw, pb = f32(300, 96), f32(5376, 96), f32(5376)
+    hx, hw = rand_bf16(rng, 300 * 5376), rand_bf16(rng, 96 * 5376, 0.02)
+    nw, mod = rand_bf16(rng, 5376, 0.1, 1.0), rand_bf16(rng, 8 * 5376, 0.1)
+    hb, rm = rand_bf16(rng, 96), rng.integers(0, 4, 300).astype(np.uint32)
+
+    def results(g):
+        o, p = g.new_f32(m * n), g.new_bf16(300 * 5376)
+        y, inv = g.new_bf16(300 * 96), g.new_f32(300)
+        g.run("h3_gpu_linear_f32", o, g.f32(x), g.f32(w), g.f32(b), m, k, n)
+        g.run("h3_gpu_patch_linear_bf16_offset", p, 0, g.f32(px), 0,
+              g.f32(pw), g.f32(pb), 300, 96, 5376)
+        g.run("h3_gpu_adaln_linear_bf16", y, inv, g.bf16(hx), 0, g.bf16(nw),
+              g.bf16(mod), g.u32(rm), g.bf16(hw), g.bf16(hb), 300, 5376, 96,
+              2, 0, 1, C.c_float(1e-5))
+        return (g.read_f32(o), g.read_bf16(p), g.read_bf16(y),
+                g.read_f32(inv))
+
+    fast = results(gpu)
+    monkeypatch.setenv("H3_HIP_REFERENCE", "1")
+    with h3hip.Gpu() as g:
+        simple = results(g)
+    terms = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    bound = 2 * (k + 16) * 2.0 ** -24 * (terms + np.abs(b))
+    d = np.abs(fast[0].astype(np.float64) - simple[0])
+    assert (d <= bound.ravel()).all()
+    np.testing.assert_array_equal(fast[1], simple[1])
+    assert_close(fast[2], simple[2], what="head", chained=1)
+    np.testing.assert_allclose(fast[3], simple[3], rtol=1e-5)

@@ -25,3 +25,27 @@ def test_head_lds_limit(rows, n, width):
     assert launch.lds <= launch.lds_limit
     if launch.lds + 17 * 4 * block_rows > 64 * 1024:
         assert launch.lds_limit > 64 * 1024
+
+
+def linear_f32(m, k, n):
+    return ["h3_gpu_linear_f32", ["f32", m * n], ["f32", m * k],
+            ["f32", n * k], ["f32", n], m, k, n]
+
+
+def patch(rows, k, n):
+    return ["h3_hip_patch_linear_bf16_offset", ["bf16", rows * n], 0,
+            ["f32", rows * k], 0, ["f32", n * k], ["f32", n], rows, k, n]
+
+
+@pytest.mark.parametrize("call,kernel,simple", [
+    (linear_f32(39, 256, 5376), "hk_linear_f32_mfma<3, 3>",
+     "hk_linear_f32_kernel"),
+    (patch(1792, 96, 5376), "hk_patch_linear_mfma", "hk_patch_linear_kernel"),
+    (head(74, 5376, 32), "hk_adaln_head_mfma<2, 4>", "hk_adaln_head_kernel"),
+])
+def test_reference_switch_takes_the_simple_kernels(call, kernel, simple):
+    for flag, want in (("0", kernel), ("1", simple)):
+        (ok, error, launches), = calls_made(
+            [call], env={"H3_HIP_REFERENCE": flag})
+        assert ok, error
+        assert [l.kernel for l in launches] == [want]
