@@ -864,7 +864,7 @@ static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
     if (scratch && bytes > scratch_bytes) splits = 1;
     if (splits > 1) {
         g.partial = scratch ? scratch
-                            : (float *)hk_splitk_space(gpu, bytes);
+                            : (float *)hk_splitk_try(gpu, bytes);
         if (!g.partial) splits = 1; /* no scratch: in one piece */
     }
     const dim3 grid(wgs, splits > 1 ? splits : 1u, problems);

@@ -127,6 +127,8 @@ void *hk_workspace(struct h3_gpu *gpu, size_t bytes);
 /* Grow-only scratch for split-K partials, separate from the workspace
  * (which may hold a GEMM's input, e.g. the MLP activation). */
 void *hk_splitk_space(struct h3_gpu *gpu, size_t bytes);
+/* The same for a caller that can do without: NULL leaves no error. */
+void *hk_splitk_try(struct h3_gpu *gpu, size_t bytes);
 
 double hk_now(void);
 

@@ -212,7 +212,7 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
     if (pieces > 1) {
         g.piece_steps = (steps + pieces - 1) / pieces;
         pieces = (steps + g.piece_steps - 1) / g.piece_steps;
-        float *partial = (float *)hk_splitk_space(
+        float *partial = (float *)hk_splitk_try(
             gpu, (size_t)pieces * m * n * sizeof(float));
         if (partial) {
             g.c = partial;

@@ -112,6 +112,8 @@ static void hk_device_release(struct h3_gpu *gpu, void *data, size_t bytes) {
     }
 }
 
+/* `what` names a failed allocation in the context's error; NULL leaves the
+ * error as it is, for a caller that can do without. */
 static void *hk_grow(struct h3_gpu *gpu, void **buffer, size_t *have,
                      size_t bytes, const char *what) {
     if (!bytes) bytes = 1;
@@ -128,7 +130,7 @@ static void *hk_grow(struct h3_gpu *gpu, void **buffer, size_t *have,
     hipError_t status = hipMalloc(&fresh, capacity);
     if (status != hipSuccess) {
         (void)hipGetLastError();
-        hk_fail_hip(gpu, what, status);
+        if (what) hk_fail_hip(gpu, what, status);
         return NULL;
     }
     *buffer = fresh;
@@ -144,6 +146,10 @@ void *hk_workspace(struct h3_gpu *gpu, size_t bytes) {
 void *hk_splitk_space(struct h3_gpu *gpu, size_t bytes) {
     return hk_grow(gpu, &gpu->splitk, &gpu->splitk_bytes, bytes,
                    "split-K scratch allocation");
+}
+
+void *hk_splitk_try(struct h3_gpu *gpu, size_t bytes) {
+    return hk_grow(gpu, &gpu->splitk, &gpu->splitk_bytes, bytes, NULL);
 }
 
 /* --------------------------------------------------------------- timing */

@@ -33,7 +33,7 @@ static hipStream_t push_stream;
 
 extern "C" {
 
-/* allocations above this many bytes fail from here on */
+/* device allocations above this many bytes fail from here on */
 void fake_largest_block(size_t bytes) { largest = bytes; }
 size_t fake_syncs() { return syncs; }
 
@@ -95,15 +95,17 @@ hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int value) {
     return hipSuccess;
 }
 
-hipError_t hipMalloc(void **p, size_t bytes) {
+static hipError_t give(void **p, size_t bytes) {
     *p = nullptr;
-    if (bytes > largest) return hipErrorOutOfMemory;
     void *m = mmap(nullptr, bytes, PROT_READ | PROT_WRITE,
                    MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (m == MAP_FAILED) return hipErrorOutOfMemory;
     blocks[m] = bytes;
     *p = m;
     return hipSuccess;
+}
+hipError_t hipMalloc(void **p, size_t bytes) {
+    return bytes > largest ? hipErrorOutOfMemory : give(p, bytes);
 }
 hipError_t hipFree(void *p) {
     auto it = blocks.find(p);
@@ -114,7 +116,7 @@ hipError_t hipFree(void *p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
-    return hipMalloc(p, bytes);
+    return give(p, bytes);
 }
 hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
@@ -132,7 +134,7 @@ hipError_t hipMemGetInfo(size_t *available, size_t *total) {
 }
 hipError_t hipGetSymbolAddress(void **p, const void *symbol) {
     void *&m = symbols[symbol];
-    if (!m) (void)hipMalloc(&m, (size_t)64 << 20);
+    if (!m) (void)give(&m, (size_t)64 << 20);
     *p = m;
     return hipSuccess;
 }

@@ -38,13 +38,15 @@ def _fake():
     return out
 
 
-def calls_made(calls, env=None, largest_block=None, contexts=1):
-    """One (ok, error text, [Launch]) per call.  `largest_block`: allocations
-    of more bytes fail once the contexts and the tensors are there.  Call i is
-    made by context i % contexts."""
+def calls_made(calls, env=None, largest_block=None, at_start=None,
+               contexts=1):
+    """One (ok, error text, [Launch]) per call.  Allocations of more than
+    `largest_block` bytes fail once the contexts and the tensors are there, of
+    more than `at_start` bytes while the contexts are made.  Call i is made by
+    context i % contexts."""
     proc = subprocess.run(
         [sys.executable, os.path.abspath(__file__), _fake()],
-        input=json.dumps([calls, largest_block, contexts]), text=True,
+        input=json.dumps([calls, largest_block, at_start, contexts]), text=True,
         capture_output=True, env={**os.environ, **(env or {})}, timeout=300)
     assert proc.returncode == 0, proc.stderr[-2000:]
     return [(ok, error, [Launch(l) for l in launches])
@@ -55,8 +57,14 @@ def _child():
     fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
     sys.path.insert(0, os.path.join(ROOT, "h3.c_amd"))
     import h3hip
-    calls, largest_block, contexts = json.loads(sys.stdin.read())
+    calls, largest_block, at_start, contexts = json.loads(sys.stdin.read())
+
+    def limit(size):
+        fake.fake_largest_block(ctypes.c_size_t(-1 if size is None else size))
+
+    limit(at_start)
     gpus = [h3hip.Gpu() for _ in range(contexts)]
+    limit(None)
     made, ready = [], []
     for i, (name, *args) in enumerate(calls):
         gpu = gpus[i % contexts]
@@ -72,14 +80,14 @@ def _child():
                 made.append(a)
             values.append(a)
         ready.append((gpu, name, values))
-    if largest_block is not None:
-        fake.fake_largest_block(ctypes.c_size_t(largest_block))
+    limit(largest_block)
     out = []
     for gpu, name, values in ready:
         fake.fake_clear()
         gpu.begin()
         ok = getattr(gpu.L, name)(gpu.h, *values)
         error = gpu.error()
+        error = "" if error == "unknown HIP error" else error  # none left
         gpu.submit()
         launches = []
         for i in range(fake.fake_launches()):

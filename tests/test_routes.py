@@ -49,3 +49,29 @@ def test_reference_switch_takes_the_simple_kernels(call, kernel, simple):
             [call], env={"H3_HIP_REFERENCE": flag})
         assert ok, error
         assert [l.kernel for l in launches] == [want]
+
+
+MIB = 1 << 20
+
+
+def linear(m, k, n, fn="h3_gpu_linear_bf16"):
+    return [fn, ["bf16", m * n], ["bf16", m * k], ["bf16", n * k], None, m, k,
+            n]
+
+
+@pytest.mark.parametrize("call,kernels,pieces", [
+    (linear(128, 14336, 128),
+     ["hk_gemm_skinny<4, 3>", "hk_skinny_reduce"], 1),
+    (linear_f32(101, 5376, 2688),
+     ["hk_linear_f32_mfma<8, 1>", "hk_linear_f32_reduce"], 2),
+])
+def test_no_scratch_takes_one_piece_and_leaves_no_error(call, kernels,
+                                                        pieces):
+    """`pieces`: the grid's dimension that counts the pieces of K."""
+    for limit in (None, MIB // 2):
+        (ok, error, launches), = calls_made([call], largest_block=limit,
+                                            at_start=limit)
+        assert ok and not error, error
+        assert (launches[0].grid[pieces] > 1) == (limit is None)
+        assert [l.kernel for l in launches] == kernels[:len(launches)]
+        assert len(launches) == (2 if limit is None else 1)
