@@ -954,9 +954,20 @@ int hk_attention_bf16(struct h3_gpu *gpu, const uint16_t *q,
         }
         const size_t part_bytes = parts * qb_rows * (HK_HD + 2) * sizeof(float);
         if (table_bytes + keys_bytes + part_bytes) {
-            uint8_t *buf = (uint8_t *)hk_splitk_space(
-                gpu, table_bytes + keys_bytes + part_bytes);
-            if (!buf) return 0;
+            uint8_t *buf = NULL;
+            if (parts) {
+                buf = (uint8_t *)hk_splitk_try(
+                    gpu, table_bytes + keys_bytes + part_bytes);
+                if (!buf) { /* no scratch for pieces: whole items */
+                    pieces = 1;
+                    parts = 0;
+                }
+            }
+            if (rope && !buf) {
+                buf = (uint8_t *)hk_splitk_space(gpu,
+                                                 table_bytes + keys_bytes);
+                if (!buf) return 0;
+            }
             if (rope) {
                 a.rope_pk = (const uint64_t *)buf;
                 const uint32_t count = q_rows * HK_ROPE_HALF;

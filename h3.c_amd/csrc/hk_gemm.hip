@@ -931,20 +931,21 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
          * does). */
         const hk_gemm_rounds r =
             hk_gemm_rounds_of(g.tile_count, k_steps, cus, true);
+        float *partial = NULL;
         if (r.splits > 1) {
-            const uint32_t full = r.full, tail = r.tail;
-            const uint32_t splits = r.splits, steps = r.steps;
             const size_t partial_bytes =
-                (size_t)splits * tail * g.tile_rows * HK_BN * 4;
+                (size_t)r.splits * r.tail * g.tile_rows * HK_BN * 4;
             if (scratch && partial_bytes > scratch_bytes)
                 return hk_fail(gpu,
                                "linear needs %zu bytes of split-K scratch, "
                                "over the %zu-byte static maximum",
                                partial_bytes, scratch_bytes);
-            float *partial = scratch ? scratch
-                                     : (float *)hk_splitk_space(
-                                           gpu, partial_bytes);
-            if (!partial) return 0;
+            partial = scratch ? scratch
+                              : (float *)hk_splitk_try(gpu, partial_bytes);
+        }
+        if (partial) { /* without scratch, the tail is one more round */
+            const uint32_t full = r.full, tail = r.tail;
+            const uint32_t splits = r.splits, steps = r.steps;
             if (full) {
                 g.tile_count = full;
                 hk_gemm_launch(gpu, hk_gemm_pick_epi(epilogue, jb), jb,

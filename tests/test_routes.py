@@ -75,3 +75,43 @@ def test_no_scratch_takes_one_piece_and_leaves_no_error(call, kernels,
         assert (launches[0].grid[pieces] > 1) == (limit is None)
         assert [l.kernel for l in launches] == kernels[:len(launches)]
         assert len(launches) == (2 if limit is None else 1)
+
+
+def attention(rows, heads):
+    n = rows * heads * 128
+    return ["h3_gpu_sdpa_bf16", *[["bf16", n]] * 4, rows, heads, 128, 0.088]
+
+
+def attention_rope(rows, heads):
+    n = rows * heads * 128
+    return ["h3_hip_sdpa_rope_bf16", *[["bf16", n]] * 4,
+            *[["bf16", rows * 48]] * 2, rows, heads, 128, 48, 0.088]
+
+
+@pytest.mark.parametrize("call,limit,kernels,whole,grid", [
+    (linear(512, 14336, 5376), 0,
+     ["hk_gemm_mfma<3, false>", "hk_splitk_reduce<0>"],
+     ["hk_gemm_mfma<0, false>"], 48),  # 42 tiles, in eights
+    (linear(9720, 5120, 13824), 0,
+     ["hk_gemm_mfma<0, false>", "hk_gemm_mfma<3, false>",
+      "hk_splitk_reduce<0>"], ["hk_gemm_mfma<0, false>"],
+     232),                             # 2052 tiles in nine rounds
+    (attention(2378, 56), 0,
+     ["hk_flash_fwd<false, false, 8>", "hk_flash_fwd<false, true, 8>",
+      "hk_flash_combine<256u>"], ["hk_flash_fwd<false, false, 8>"], 560),
+    # the rotated keys still need theirs, 50 of 67 MiB (blocks double)
+    (attention_rope(3584, 56), 64 * MIB,
+     ["hk_rope_pack", "hk_rope_keys", "hk_flash_fwd<false, false, 8>",
+      "hk_flash_fwd<false, true, 8>", "hk_flash_combine<256u>"],
+     ["hk_rope_pack", "hk_rope_keys", "hk_flash_fwd<false, false, 8>"],
+     784),
+])
+def test_no_scratch_runs_whole(call, limit, kernels, whole, grid):
+    """Tiles and attention items that would be cut run whole where scratch for
+    the pieces cannot be had."""
+    for largest, want in ((None, kernels), (limit, whole)):
+        (ok, error, launches), = calls_made([call], largest_block=largest,
+                                            at_start=largest)
+        assert ok and not error, error
+        assert [l.kernel for l in launches] == want
+    assert launches[-1].grid == [grid, 1, 1]
