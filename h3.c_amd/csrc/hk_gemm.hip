@@ -835,12 +835,15 @@ static void hk_skinny_lds_setup(const struct h3_gpu *gpu) {
     ready |= bit;
 }
 
-/* Launches hk_gemm_skinny: `problems` of them from a table, or one. */
+/* Launches hk_gemm_skinny: `problems` of them from a table, or one.  The
+ * pieces' sums, at most 64 KiB a CU, go to the context's scratch, which has
+ * room for them from its creation: a call that may not allocate finds it
+ * there, and calls of two contexts share nothing. */
 static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
                               const uint16_t *w, const uint16_t *bias,
                               uint16_t *c, uint32_t m, uint32_t n, uint32_t k,
                               const uint64_t *group, uint32_t problems,
-                              float *scratch, size_t scratch_bytes) {
+                              bool may_allocate) {
     const uint32_t mbs = (m + 31u) / 32u, wgs = (n + 127u) / 128u;
     const uint32_t k_steps = k / HK_BK;
     hk_skinny_args g;
@@ -859,12 +862,12 @@ static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
         g.split_steps = ((k_steps + splits - 1) / splits + 3u) & ~3u;
         splits = (k_steps + g.split_steps - 1) / g.split_steps;
     }
-    const size_t bytes = (size_t)splits * wgs * 4 * mbs * 4096;
-    /* at most a 64-KiB piece per CU: a quarter of the no-alloc scratch */
-    if (scratch && bytes > scratch_bytes) splits = 1;
     if (splits > 1) {
-        g.partial = scratch ? scratch
-                            : (float *)hk_splitk_try(gpu, bytes);
+        const size_t bytes = (size_t)splits * wgs * 4 * mbs * 4096;
+        if (may_allocate)
+            g.partial = (float *)hk_splitk_try(gpu, bytes);
+        else if (bytes <= gpu->splitk_bytes)
+            g.partial = (float *)gpu->splitk;
         if (!g.partial) splits = 1; /* no scratch: in one piece */
     }
     const dim3 grid(wgs, splits > 1 ? splits : 1u, problems);
@@ -895,7 +898,7 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
     const bool mfma = hk_gemm_mfma_ok(gpu, x, w, bias, c, m, n, k, epilogue);
     if (mfma && epilogue == HK_EPI_STORE && hk_skinny_ok(m, n, k))
         return hk_gemm_skinny_run(gpu, x, w, bias, c, m, n, k, NULL, 1,
-                                  scratch, scratch_bytes);
+                                  scratch == NULL);
     if (mfma) {
         hk_gemm_lds_setup(gpu);
         hk_gemm_args g;
@@ -1062,7 +1065,7 @@ static int hk_gemm_bf16_group(struct h3_gpu *gpu, const uint16_t *x,
         for (uint32_t p = 0; p < count; p += 65535u)
             if (!hk_gemm_skinny_run(gpu, x, NULL, NULL, NULL, m, n, k,
                                     table + (size_t)p * 3,
-                                    min(count - p, 65535u), NULL, 0))
+                                    min(count - p, 65535u), true))
                 return 0;
         return 1;
     }
@@ -1089,7 +1092,7 @@ static int hk_gemm_bf16_group(struct h3_gpu *gpu, const uint16_t *x,
 
 /* ================================================== allocation-free linear
  *
- * h3_hip_linear_bf16_noalloc's split-K partials live in this file-scope
+ * h3_hip_linear_bf16_noalloc's split-K partial tiles live in this file-scope
  * device array instead of the context's on-demand scratch, so the call
  * makes no allocation.  Each device holds its own copy from the library's
  * load until the process ends; its address on a device comes from

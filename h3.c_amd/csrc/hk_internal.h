@@ -127,6 +127,9 @@ void *hk_workspace(struct h3_gpu *gpu, size_t bytes);
 /* Grow-only scratch for split-K partials, separate from the workspace
  * (which may hold a GEMM's input, e.g. the MLP activation). */
 void *hk_splitk_space(struct h3_gpu *gpu, size_t bytes);
+/* A context's split-K scratch starts with this much a CU: the most that the
+ * pieces of a launch of at most 128 rows need (128 x 128 F32 sums). */
+enum { HK_SKINNY_CU_BYTES = 64 * 1024 };
 /* The same for a caller that can do without: NULL leaves no error. */
 void *hk_splitk_try(struct h3_gpu *gpu, size_t bytes);
 
@@ -146,7 +149,8 @@ enum { HK_EPI_STORE = 0, HK_EPI_SWIGLU = 1, HK_EPI_GELU = 2,
  * 2*N rows (gate rows [0,N), up rows [N,2N)) and C is the [M,N] activation.
  * Split-K partials go to the context's scratch (grown on demand), or, when
  * `scratch` is given, to that caller-owned device buffer of scratch_bytes:
- * then nothing is allocated, and a split that needs more fails. */
+ * then nothing is allocated, and a split that needs more fails (launches of
+ * at most 128 rows use what the context has, and need no buffer). */
 int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *a, const uint16_t *w,
                  const uint16_t *bias, uint16_t *c, uint32_t m, uint32_t n,
                  uint32_t k, int epilogue, float *scratch = nullptr,

@@ -380,6 +380,8 @@ extern "C" h3_gpu *h3_gpu_create(const char *shader_source_path,
     if (hipGetDeviceProperties(&properties, 0) == hipSuccess)
         gpu->num_cus = properties.multiProcessorCount;
     if (gpu->num_cus <= 0) gpu->num_cus = 256;
+    /* the skinny GEMM's pieces (their calls do without where refused) */
+    (void)hk_splitk_try(gpu, (size_t)gpu->num_cus * HK_SKINNY_CU_BYTES);
     gpu->reference_kernels = hk_env_flag("H3_HIP_REFERENCE");
     gpu->profile_mark_wall = hk_now();
     if (!hk_loader_new(gpu)) {

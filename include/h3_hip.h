@@ -227,13 +227,15 @@ int h3_hip_linear_pair_bf16(h3_gpu *gpu, h3_gpu_tensor *output0,
                             uint32_t input_dim, uint32_t output_dim);
 
 /* h3_gpu_linear_bf16 that allocates nothing: the same kernels and the same
- * results, with the split-K partial sums (used when the last round of tiles,
- * or a launch of at most 128 rows, would leave CUs idle) in a static 64 MiB
- * device array per GPU instead of the context's on-demand scratch.  A
+ * results.  At most 128 rows: the pieces' partial sums go to scratch that the
+ * context holds from its creation (64 KiB a CU), and calls of several
+ * contexts may overlap.  More rows: the split-K partial tiles (used when the
+ * last round of tiles would leave over half the CUs idle) go to a static 64
+ * MiB device array per GPU instead of the context's on-demand scratch.  A
  * launch whose split would need more fails with an error naming the size.
  * The array (256 CUs x one 256x256 f32 tile) is resident on every GPU the
- * library loads on, whether or not this entry is called.  Calls that
- * overlap on one GPU share that array and race.  No counterpart in the
+ * library loads on, whether or not this entry is called.  Calls of more than
+ * 128 rows that overlap on one GPU share that array and race.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory
  * (fixed-footprint serving loops, harnesses that forbid hipMalloc); it
  * makes no device allocation, but recording it into a HIP graph is not

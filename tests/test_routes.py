@@ -115,3 +115,22 @@ def test_no_scratch_runs_whole(call, limit, kernels, whole, grid):
         assert ok and not error, error
         assert [l.kernel for l in launches] == want
     assert launches[-1].grid == [grid, 1, 1]
+
+
+@pytest.mark.parametrize("rows", [8, 40, 64, 128])
+def test_noalloc_pieces_of_two_contexts_share_nothing(rows):
+    """Few rows: each context's pieces have scratch of its own, held since its
+    creation, so that calls of two contexts may overlap."""
+    fn = "h3_hip_linear_bf16_noalloc"
+    made = calls_made([linear(rows, 14336, 5376, fn),
+                       linear(rows, 14336, 5376, fn)], contexts=2,
+                      largest_block=0)
+    partial = []
+    for ok, error, launches in made:
+        assert ok and not error, error
+        assert [l.kernel for l in launches][1:] == ["hk_skinny_reduce"]
+        assert launches[0].grid[1] > 1
+        size = launches[0].grid[0] * launches[0].grid[1] * 65536
+        partial.append((launches[0].words[7], size))
+    (a, size_a), (b, size_b) = partial
+    assert a and b and (a + size_a <= b or b + size_b <= a)

@@ -5,6 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import h3hip
 import oracle
 from conftest import assert_close, rand_bf16
 
@@ -66,3 +67,38 @@ def test_linear_group_skinny(gpu, m, k, n, count, first):
                              what=f"group[{p}]")
     finally:
         gpu.L.h3_gpu_tensor_free(table)
+
+
+@pytest.mark.parametrize("m", [8, 64, 128])
+def test_noalloc_calls_of_two_contexts_overlap(m):
+    """Two contexts enqueue allocation-free calls in turn and submit only
+    then: each result is the one that the context gives alone."""
+    k, n, calls = 14336, 1280, 8
+    rng = np.random.default_rng(m)
+    w = rand_bf16(rng, n * k, 0.05)
+    xs = [rand_bf16(rng, m * k) for _ in range(2)]
+    gpus = [h3hip.Gpu() for _ in xs]
+    try:
+        tw = [g.bf16(w) for g in gpus]
+        tx = [g.bf16(x) for g, x in zip(gpus, xs)]
+        outs = [[g.new_bf16(m * n) for _ in range(calls)] for g in gpus]
+        alone = []
+        for g, x, t, o in zip(gpus, tx, tw, outs):
+            g.run("h3_gpu_linear_bf16", o[0], x, t, None, m, k, n)
+            alone.append(g.read_bf16(o[0]))
+            assert_close(alone[-1], oracle.linear(xs[len(alone) - 1], w, None,
+                                                  m, k, n), what="alone")
+        for g in gpus:
+            g.begin()
+        for c in range(calls):
+            for g, x, t, o in zip(gpus, tx, tw, outs):
+                g.check(g.L.h3_hip_linear_bf16_noalloc(
+                    g.h, o[c], x, t, None, m, k, n), "noalloc")
+        for g in gpus:
+            g.submit()
+        for g, o, want in zip(gpus, outs, alone):
+            for t in o:
+                assert np.array_equal(g.read_bf16(t), want)
+    finally:
+        for g in gpus:
+            g.close()
