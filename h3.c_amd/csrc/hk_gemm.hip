@@ -390,7 +390,7 @@ hk_gemm_skinny(hk_skinny_args g) {
 #pragma unroll
         for (int i = 0; i < MB; i++)
             hk_dma16(xr, hk_xs + buf * XSTAGE + (256u * i + wave * 64u) * 16u,
-                     xo[i] | hk_skinny_dead(step, steps),
+                     hk_skinny_lane(xo[i], step, steps),
                      hk_skinny_k_bytes(base + step, k / 64u));
     };
     hk_v4i wf[D][4];
@@ -398,7 +398,7 @@ hk_gemm_skinny(hk_skinny_args g) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
             wf[slot][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                wr, wo[q] | hk_skinny_dead(step, steps),
+                wr, hk_skinny_lane(wo[q], step, steps),
                 hk_skinny_k_bytes(base + step, k / 64u), HK_LOAD_ONCE);
     };
     /* fragment of X rows mb*32 + row, logical chunk 2q + half */
@@ -816,14 +816,6 @@ static uint32_t hk_gemm_row_blocks(uint32_t m, uint32_t columns,
     return best;
 }
 
-/* Whether a shape that hk_gemm_mfma_ok takes is one for hk_gemm_skinny. */
-static bool hk_skinny_ok(uint32_t m, uint32_t n, uint32_t k) {
-    const uint64_t margin = 4ull * k + 4096;
-    return m <= HK_SKINNY_ROWS &&
-           (uint64_t)n * k * 2 + margin < HK_SKINNY_LIMIT &&
-           (uint64_t)m * k * 2 + margin < HK_SKINNY_LIMIT;
-}
-
 /* 80 KiB of dynamic LDS need the kernel's limit raised, once per device. */
 static void hk_skinny_lds_setup(const struct h3_gpu *gpu) {
     static uint64_t ready = 0;
@@ -896,7 +888,7 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
     const uint64_t w_rows = epilogue == HK_EPI_SWIGLU ? 2ull * n : n;
     const uint64_t x_bytes = (uint64_t)m * k * 2, w_bytes = w_rows * k * 2;
     const bool mfma = hk_gemm_mfma_ok(gpu, x, w, bias, c, m, n, k, epilogue);
-    if (mfma && epilogue == HK_EPI_STORE && hk_skinny_ok(m, n, k))
+    if (mfma && epilogue == HK_EPI_STORE && m <= HK_SKINNY_ROWS)
         return hk_gemm_skinny_run(gpu, x, w, bias, c, m, n, k, NULL, 1,
                                   scratch == NULL);
     if (mfma) {
@@ -1014,7 +1006,7 @@ int hk_gemm_bf16_pair(struct h3_gpu *gpu, const uint16_t *x,
     const uint32_t tiles = ((m + HK_BM - 1) / HK_BM) * ((n + HK_BN - 1) / HK_BN);
     const uint32_t k_steps = k / HK_BK;
     const bool paired =
-        !hk_skinny_ok(m, n, k) && k_steps >= 8 && tiles * 4 <= cus &&
+        m > HK_SKINNY_ROWS && k_steps >= 8 && tiles * 4 <= cus &&
         hk_gemm_mfma_ok(gpu, x, w0, b0, c0, m, n, k, HK_EPI_STORE) &&
         hk_gemm_mfma_ok(gpu, x, w1, b1, c1, m, n, k, HK_EPI_STORE);
     if (!paired)
@@ -1060,7 +1052,7 @@ static int hk_gemm_bf16_group(struct h3_gpu *gpu, const uint16_t *x,
                               const uint64_t *table, uint32_t count,
                               uint32_t m, uint32_t n, uint32_t k) {
     if (!m || !n || !count) return 1;
-    if (hk_skinny_ok(m, n, k)) {
+    if (m <= HK_SKINNY_ROWS) {
         /* a grid's z dimension ends at 65535 */
         for (uint32_t p = 0; p < count; p += 65535u)
             if (!hk_gemm_skinny_run(gpu, x, NULL, NULL, NULL, m, n, k,

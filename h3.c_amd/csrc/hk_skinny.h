@@ -16,17 +16,16 @@
  * the ring they go round in */
 enum { HK_SKINNY_RING = 4 };
 
-/* the operands' bytes stay below this bit, which marks a dead offset */
-#define HK_SKINNY_LIMIT 0x80000000u
-
 /* The scalar offset of k step `step` of `k_steps`. */
 constexpr uint32_t hk_skinny_k_bytes(uint32_t step, uint32_t k_steps) {
     return (step < k_steps ? step : k_steps - 1u) * 128u;
 }
 
-/* Set in the lane offsets of a step past the end of its piece. */
-constexpr uint32_t hk_skinny_dead(uint32_t step, uint32_t piece_steps) {
-    return step < piece_steps ? 0u : HK_SKINNY_LIMIT;
+/* The lane offset of a load: `offset`, or past any operand (whose bytes end
+ * 2 K + 4096 below 2^32) for a step past the end of its piece. */
+constexpr uint32_t hk_skinny_lane(uint32_t offset, uint32_t step,
+                                  uint32_t piece_steps) {
+    return step < piece_steps ? offset : 0xfffff000u;
 }
 
 #endif

@@ -134,3 +134,13 @@ def test_noalloc_pieces_of_two_contexts_share_nothing(rows):
         partial.append((launches[0].words[7], size))
     (a, size_a), (b, size_b) = partial
     assert a and b and (a + size_a <= b or b + size_b <= a)
+
+
+@pytest.mark.parametrize("rows,kernel", [(39, "hk_gemm_skinny<2, 1>"),
+                                         (128, "hk_gemm_skinny<4, 3>")])
+def test_few_rows_take_the_skinny_kernel_with_any_weight(rows, kernel):
+    """Any weight that the GEMMs take (up to 4 GiB)."""
+    for n in (5376, 420000, 780000):  # 29 MB, 2.3 GB, 4.2 GB
+        (ok, error, launches), = calls_made([linear(rows, 2688, n)])
+        assert ok, error
+        assert launches[0].kernel in (kernel, kernel[:-2] + "3>")

@@ -102,3 +102,23 @@ def test_noalloc_calls_of_two_contexts_overlap(m):
     finally:
         for g in gpus:
             g.close()
+
+
+def test_skinny_weight_over_two_gib(gpu):
+    """The first and the last columns of a weight past 2 GiB, each block
+    copied out and multiplied by the oracle."""
+    m, k, n, block = 40, 2688, 420004, 68
+    rng = np.random.default_rng(12)
+    x = rand_bf16(rng, m * k)
+    w, out, part = (gpu.new_bf16(s) for s in (n * k, m * n, block * k))
+    gpu.run("h3_gpu_fill_normal_bf16", w, 0, n * k, 3, C.c_float(0.0),
+            C.c_float(0.05))
+    gpu.run("h3_gpu_linear_bf16", out, gpu.bf16(x), w, None, m, k, n)
+    got = gpu.read_bf16(out).reshape(m, n)
+    for first in (0, (1 << 30) // k - 30, n - block):
+        gpu.run("h3_gpu_copy_bf16", part, 0, w, first * k, block * k)
+        want = oracle.linear(x, gpu.read_bf16(part), None, m, k, block)
+        assert_close(got[:, first:first + block].ravel(), want,
+                     what=f"columns from {first}")
+    for t in (w, out, part):
+        gpu.free(t)

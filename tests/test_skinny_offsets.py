@@ -15,12 +15,14 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 WALK = r"""
 #include <stdio.h>
+#include <initializer_list>
 #include "hk_skinny.h"
 static int bad;
-/* rows x k operand, of which the kernel asks for `asked` rows (those past the
- * end as row `rows`), in pieces of `piece` k steps loaded up to `ahead` ahead */
+/* rows x k operand, of which the kernel asks for rows from `first` to `asked`
+ * (those past the end as row `rows`), in pieces of `piece` k steps loaded up
+ * to `ahead` ahead */
 static void walk(uint32_t rows, uint32_t asked, uint32_t k, uint32_t piece,
-                 uint32_t ahead) {
+                 uint32_t ahead, uint32_t first = 0) {
     const uint32_t bytes = rows * k * 2, k_steps = k / 64;
     for (uint32_t base = 0; base < k_steps; base += piece) {
         const uint32_t steps =
@@ -29,11 +31,11 @@ static void walk(uint32_t rows, uint32_t asked, uint32_t k, uint32_t piece,
             (steps + HK_SKINNY_RING - 1) / HK_SKINNY_RING * HK_SKINNY_RING;
         for (uint32_t s = 0; s < turns + ahead; s++) {
             const uint32_t at = hk_skinny_k_bytes(base + s, k_steps);
-            const uint32_t dead = hk_skinny_dead(s, steps);
-            for (uint32_t r = 0; r < asked; r++)
+            for (uint32_t r = first; r < asked; r++)
                 for (uint32_t chunk = 0; chunk < 8; chunk++) {
                     const uint32_t row = r < rows ? r : rows;
-                    const uint32_t lane = (row * k * 2 + chunk * 16) | dead;
+                    const uint32_t lane =
+                        hk_skinny_lane(row * k * 2 + chunk * 16, s, steps);
                     const bool passes = lane < bytes - at; /* unsigned */
                     const bool wanted = r < rows && s < steps;
                     if (at >= bytes || passes != wanted ||
@@ -56,6 +58,14 @@ int main() {
                 walk(r, 64, k_steps * 64, piece, 1); /* X, one or three */
                 walk(r, 64, k_steps * 64, piece, 3); /* steps ahead; W */
             }
+    /* the largest W that the GEMMs take: 2 K + 4096 bytes below 2^32 */
+    for (uint32_t k_steps : {1u, 2u, 3u, 42u, 84u, 224u}) {
+        const uint32_t k = k_steps * 64;
+        const uint32_t rows = (uint32_t)((0xffffffffull - 4096 - 2 * k) /
+                                         (2 * k)) & ~3u;
+        for (uint32_t piece = 4; piece < k_steps + 4; piece += 4)
+            walk(rows, rows + 128, k, piece, 3, rows - 8);
+    }
     if (bad) printf("%d loads\n", bad);
     return bad != 0;
 }
