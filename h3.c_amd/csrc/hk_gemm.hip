@@ -694,7 +694,12 @@ static hk_gemm_kernel hk_gemm_pick(uint32_t jb) {
     case 4: return hk_gemm_mfma_low<EPI, GROUP, 4>;
     case 5: return hk_gemm_mfma_low<EPI, GROUP, 5>;
     case 6: return hk_gemm_mfma_low<EPI, GROUP, 6>;
-    case 7: return hk_gemm_mfma_low<EPI, GROUP, 7>;
+    case 7:
+        /* no plan cuts 224-row tiles (hk_gemm_row_blocks) */
+        if constexpr (EPI == HK_EPI_PARTIAL || EPI == HK_EPI_PARTIAL_SWIGLU)
+            return NULL;
+        else
+            return hk_gemm_mfma_low<EPI, GROUP, 7>;
     default: return hk_gemm_mfma<EPI, GROUP>;
     }
 }
@@ -719,10 +724,11 @@ static void hk_gemm_lds_setup(const struct h3_gpu *gpu) {
     if (hk_gemm_lds_ready & bit) return;
     for (uint32_t jb = 4; jb <= 8; jb++) {
         for (int epi = HK_EPI_STORE; epi <= HK_EPI_PARTIAL_SWIGLU; epi++)
-            (void)hipFuncSetAttribute(
-                (const void *)hk_gemm_pick_epi(epi, jb),
-                hipFuncAttributeMaxDynamicSharedMemorySize,
-                (int)hk_gemm_lds(jb));
+            if (const hk_gemm_kernel kernel = hk_gemm_pick_epi(epi, jb))
+                (void)hipFuncSetAttribute(
+                    (const void *)kernel,
+                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                    (int)hk_gemm_lds(jb));
         (void)hipFuncSetAttribute(
             (const void *)hk_gemm_pick<HK_EPI_STORE, true>(jb),
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)hk_gemm_lds(jb));
@@ -782,33 +788,65 @@ static float hk_gemm_estimate(uint32_t jb, uint32_t tiles, uint32_t k_steps,
     return (float)rounds * round(k_steps, (tiles + rounds - 1) / rounds);
 }
 
-/* The tile height, in 32-row units, for m rows in `columns` column tiles:
- * the one with the lowest estimate.  256 rows use the fewest cycles and bytes
- * per flop, but pad 300 rows by 70% and 1300 by 18%, and another height can
- * fill the last round of CUs: measured (us, 256 rows against the pick) 114
- * and 100 for 300 x 5376 -> 21504, 190 and 173 for 778 x the same, 145 and
- * 115 for 1600 x 7168 -> 5376, 316 and 288 for 2378 x 14336 -> 5376.  Where
- * every tile is split along K, more row tiles read the weights more often
- * (512 x 14336 -> 5376: 88 us with 256 rows, 121 with 128), which the
- * estimate leaves out, and 224 rows gained nothing: there only 160 and 192
- * rows in as many row tiles count. */
+/* The tile height, in 32-row units, for m rows in `columns` column tiles.
+ * 256 rows use the fewest cycles and bytes per flop, but pad 300 rows by 70%
+ * and 1600 by 12%.  A lower height replaces them where the estimate gains and
+ * the launch keeps its form, as timed in turn near the power cap (344 sizes of
+ * the two models, 140-9720 rows, every height; the rule takes 2.6% of the
+ * 3.4% that the best heights give and loses over 1% nowhere that a second
+ * run bore out):
+ * - in as many rounds of CUs and with no cut tail.  More rounds never won
+ *   (the H3 MLP of 1400 rows with 160-row SwiGLU tiles, 4 rounds for 3: 571
+ *   and 630 us), and a cut tail after them costs more than the estimate says
+ *   (778 x 5376 -> 21504 with 128 rows: 186 and 275 us);
+ * - with no band of a single row tile at the end, which streams all of W for
+ *   one tile each (2000 x 5120 -> 13824 in nine row tiles of 224: 238 and
+ *   254 us).
+ * The gain has to be over 2%, and over 5%, the estimate's error there, if the
+ * 256-row tiles end in a cut tail and the lower ones need several bands (6144
+ * x 5120 -> 13824: 0.5% by the estimate, 688 and 696 us with 224 rows).
+ * Measured (us, 256 rows and the pick): 300 x 5376 -> 21504 111 and 100, 778
+ * 186 and 176; 1600 x 7168 -> 5376 130 and 114; 2378 x 14336 -> 5376 304 and
+ * 286.
+ * Where every tile is cut along K, more row tiles read the weights more often
+ * (512 x 14336 -> 5376: 89 us with 256 rows, 114 with 192): there 128, 160 and
+ * 192 rows in as many row tiles count.  Of a long K (over 8192) they gain
+ * nothing in one row tile (140 x 13824 -> 5120: 52 and 53 us), nor if the
+ * pieces cannot be dealt to the XCDs in eights (300 x 14336 -> 5376, 252
+ * pieces: 79 and 82 us; 350 x 13824 -> 5120, 240 pieces: 70 and 64). */
 static uint32_t hk_gemm_row_blocks(uint32_t m, uint32_t columns,
                                    uint32_t k_steps, uint32_t cus,
                                    bool may_split) {
     const uint32_t high = (m + HK_BM - 1) / HK_BM;
     const hk_gemm_rounds r =
         hk_gemm_rounds_of(high * columns, k_steps, cus, may_split);
-    const bool all_split = r.splits > 1 && !r.full;
+    const bool cut = r.splits > 1, all_cut = cut && !r.full;
+    const uint32_t rounds = (high * columns + cus - 1) / cus;
+    if (all_cut && k_steps > 128 &&
+        (high == 1 || r.tail * r.splits % 8u))
+        return 8;
+    const float base =
+        hk_gemm_estimate(8, high * columns, k_steps, cus, may_split);
     uint32_t best = 8;
-    /* 1% in favour of the 256-row kernel */
-    float least =
-        0.99f * hk_gemm_estimate(8, high * columns, k_steps, cus, may_split);
+    float least = base;
     for (uint32_t jb = 7; jb >= 4; jb--) {
         const uint32_t tiles_m = (m + 32u * jb - 1) / (32u * jb);
-        if (all_split && (tiles_m > high || jb == 7)) continue;
-        const float us = hk_gemm_estimate(jb, tiles_m * columns, k_steps, cus,
-                                          may_split);
-        if (us < least) {
+        const uint32_t tiles = tiles_m * columns;
+        float margin;
+        if (all_cut) {
+            if (tiles_m > high || jb == 7) continue;
+            margin = 0.01f;
+        } else {
+            if ((tiles + cus - 1) / cus != rounds ||
+                (tiles_m > HK_GROUP_M && tiles_m % HK_GROUP_M == 1) ||
+                hk_gemm_rounds_of(tiles, k_steps, cus, may_split).splits > 1)
+                continue;
+            margin = !cut                    ? 0.02f
+                     : tiles_m <= HK_GROUP_M ? 0.0f
+                                             : 0.05f;
+        }
+        const float us = hk_gemm_estimate(jb, tiles, k_steps, cus, may_split);
+        if (us < least && us < (1.0f - margin) * base) {
             best = jb;
             least = us;
         }

@@ -94,7 +94,8 @@ def test_linear_repeats_bit_exactly(gpu, m, k, n, bias, mlp):
     (512, 5120, 5120, True),    # split-K: Wan cross K/V projection (40 tiles)
     (260, 2048, 516, True),     # split-K, ragged M and N, 4 splits
     (600, 1088, 256, False),    # split-K with a short last split (17 steps)
-    (4096, 512, 4352, True),    # 272 tiles: one full round + a split tail
+    (4096, 512, 4352, True),    # 442 160-row tiles in two rounds
+    (1292, 512, 22980, True),   # 540 tiles: two full rounds + a split tail
     (4100, 256, 4200, True),    # 289 tiles, full round with ragged M and N
     (300, 64, 520, True),       # one K stage: loads and prefetch clamp to it
     (2378, 128, 1000, False),   # two K stages, H3 rows, ragged N
@@ -309,8 +310,9 @@ def test_linear_stats_kind(gpu):
     (64, 256, 512),       # 4 SwiGLU tiles, too few K steps to split
     (300, 1024, 1536),    # 24 tiles, cut along K (SwiGLU split-K reduce)
     (130, 5376, 512),     # 4 tiles at the real hidden size, 21 splits
-    (300, 512, 4608),     # 72 tiles, 2 splits
-    (300, 512, 17408),    # 272 tiles: one full round + a 16-tile split tail
+    (300, 512, 4608),     # 72 160-row tiles, 2 splits
+    (300, 512, 17408),    # 408 128-row tiles in two rounds
+    (64, 512, 33280),     # 260 tiles: one full round + a 4-tile split tail
 ])
 def test_mlp_swiglu(gpu, rows, d, ffn):
     rng = np.random.default_rng(rows + d + ffn)
@@ -325,9 +327,9 @@ def test_mlp_swiglu(gpu, rows, d, ffn):
 
 
 def test_linear_gelu_full_round_and_split_tail(gpu):
-    """272 tiles on 256 CUs: the first 256 run whole, the last 16 are cut
+    """540 tiles on 256 CUs: the first 512 run whole, the last 28 are cut
     along K and reduced with the bias and GELU."""
-    m, k, n = 4096, 640, 4352
+    m, k, n = 1292, 640, 22980
     rng = np.random.default_rng(17)
     x = rand_bf16(rng, m * k)
     w = rand_bf16(rng, n * k, 0.05)
@@ -703,10 +705,10 @@ def test_qkv_in_place_rejects_other_shapes(gpu):
 
 @pytest.mark.parametrize("q_rows,kv_rows,heads", [
     (100, 100, 2),      # reference test_cuda_attention.c hd128 N=100
-    (300, 300, 3),      # two 256-query blocks, ragged key tail, 2 pieces
+    (300, 300, 3),      # three 128-query blocks, ragged key tail
     (64, 64, 1),        # exactly one key tile
     (1000, 1000, 2),    # 8 work items on 256 CUs: 8 key-range pieces each
-    (2378, 2378, 4),    # H3 length: 40 items, 8 pieces of 5 key tiles
+    (2378, 2378, 4),    # H3 length: 40 items, 5 pieces of 8 key tiles
     (300, 77, 2),       # cross attention, short context
     (70, 513, 2),       # cross attention, more keys than queries
 ])
@@ -732,7 +734,7 @@ def test_sdpa(gpu, q_rows, kv_rows, heads):
 
 @pytest.mark.parametrize("rows,heads", [
     (100, 2),       # one query block, ragged single key tile
-    (300, 3),       # two query blocks, ragged tail, key-split pieces
+    (300, 3),       # three 128-query blocks, ragged tail
     (1000, 2),      # 8 key-range pieces per item
     (2378, 4),      # the H3 length
 ])

@@ -1,6 +1,7 @@
 """Which kernels a call launches, on 256 CUs, without a GPU (launches.py)."""
 import pytest
 
+import test_gemm_rows_gpu as gemm_rows
 from launches import calls_made
 
 
@@ -144,3 +145,106 @@ def test_few_rows_take_the_skinny_kernel_with_any_weight(rows, kernel):
         (ok, error, launches), = calls_made([linear(rows, 2688, n)])
         assert ok, error
         assert launches[0].kernel in (kernel, kernel[:-2] + "3>")
+
+
+STORE, SWIGLU_UP, GELU_UP = 0, 1, 2
+
+
+def mlp(m, k, n):
+    return ["h3_gpu_mlp_bf16", ["bf16", m * k], ["bf16", m * k],
+            ["bf16", 2 * n * k], ["bf16", n * k], m, k, n, k]
+
+
+def gemm(m, k, n, epilogue):
+    if epilogue == SWIGLU_UP:
+        return mlp(m, k, n)
+    return linear(m, k, n, "h3_gpu_linear_gelu_bf16" if epilogue == GELU_UP
+                  else "h3_gpu_linear_bf16")
+
+
+def gemm_kernels(rows, form, epilogue):
+    def kernel(epi):
+        return (f"hk_gemm_mfma<{epi}, false>" if rows == 256 else
+                f"hk_gemm_mfma_low<{epi}, false, {rows // 32}>")
+    partial = 4 if epilogue == SWIGLU_UP else 3
+    cut = [kernel(partial), f"hk_splitk_reduce<{epilogue}>"]
+    return {gemm_rows.WHOLE: [kernel(epilogue)], gemm_rows.CUT: cut,
+            gemm_rows.TAIL: [kernel(epilogue)] + cut}[form]
+
+
+def test_gemm_sizes_take_the_tiles_they_are_listed_under():
+    """The sizes of the GPU tests: each tile height and form is reached."""
+    sizes = ([(s, e) for s in gemm_rows.LINEAR for e in (STORE, GELU_UP)] +
+             [(s, GELU_UP) for s in gemm_rows.GELU] +
+             [(s, SWIGLU_UP) for s in gemm_rows.SWIGLU])
+    made = calls_made([gemm(*s[2], e) for s, e in sizes])
+    for ((rows, form, size), e), (ok, error, launches) in zip(sizes, made):
+        want = gemm_kernels(rows, form, e)
+        assert ok, error
+        assert [l.kernel for l in launches][:len(want)] == want, size
+
+
+# (m, K, N, epilogue), rows of a tile, form
+MODEL_SIZES = [
+    # 6144 and 9720 rows of the Wan block keep 256-row tiles: 224 rows were
+    # 0.5% better by the estimate and 1.2% slower (FFN up at 6144)
+    ((6144, 5120, 13824, GELU_UP), 256, gemm_rows.TAIL),
+    ((6144, 13824, 5120, STORE), 256, gemm_rows.WHOLE),
+    ((6144, 5120, 15360, STORE), 256, gemm_rows.WHOLE),
+    ((6144, 5120, 5120, STORE), 256, gemm_rows.WHOLE),
+    ((9720, 5120, 13824, GELU_UP), 256, gemm_rows.TAIL),
+    ((9720, 13824, 5120, STORE), 256, gemm_rows.WHOLE),
+    ((9720, 5120, 15360, STORE), 256, gemm_rows.WHOLE),
+    # more rounds: 339 and 380 us with 160 rows
+    ((1400, 5376, 14336, SWIGLU_UP), 256, gemm_rows.WHOLE),
+    # a last band of one row tile: 238 and 254 us with 224 rows
+    ((2000, 5120, 13824, GELU_UP), 256, gemm_rows.WHOLE),
+    # SwiGLU of 2900-3030 rows: 192 rows gain under 1.5%
+    ((2960, 5376, 14336, SWIGLU_UP), 256, gemm_rows.TAIL),
+    # every tile cut, long K, 252 pieces: 79 and 82 us with 160 rows
+    ((300, 14336, 5376, STORE), 256, gemm_rows.CUT),
+    # gains of 5% and more
+    ((778, 5376, 21504, STORE), 160, gemm_rows.WHOLE),
+    ((1600, 7168, 5376, STORE), 160, gemm_rows.WHOLE),
+    ((2378, 14336, 5376, STORE), 224, gemm_rows.WHOLE),
+    ((1300, 5120, 15360, STORE), 192, gemm_rows.WHOLE),
+    ((350, 13824, 5120, STORE), 192, gemm_rows.CUT),
+    ((100, 5120, 13824, GELU_UP), 128, gemm_rows.CUT),
+]
+
+
+def test_gemm_tile_heights_of_the_models():
+    made = calls_made([gemm(*size) for size, _, _ in MODEL_SIZES])
+    for (size, rows, form), (ok, error, launches) in zip(MODEL_SIZES, made):
+        want = gemm_kernels(rows, form, size[3])
+        assert ok, error
+        assert [l.kernel for l in launches][:len(want)] == want, size
+
+
+# sizes of test_ops_gpu.py whose comments name a path: rows of a tile, form
+OPS_SIZES = [
+    ((300, 5376, 1024, STORE), 160, gemm_rows.CUT),
+    ((512, 5120, 5120, STORE), 256, gemm_rows.CUT),
+    ((260, 2048, 516, STORE), 256, gemm_rows.CUT),
+    ((600, 1088, 256, STORE), 256, gemm_rows.CUT),
+    ((4096, 512, 4352, STORE), 160, gemm_rows.WHOLE),
+    ((1292, 512, 22980, STORE), 256, gemm_rows.TAIL),
+    ((4100, 256, 4200, STORE), 256, gemm_rows.WHOLE),
+    ((300, 64, 520, STORE), 256, gemm_rows.WHOLE),
+    ((2378, 128, 1000, STORE), 256, gemm_rows.WHOLE),
+    ((64, 256, 512, SWIGLU_UP), 256, gemm_rows.WHOLE),
+    ((300, 1024, 1536, SWIGLU_UP), 160, gemm_rows.CUT),
+    ((130, 5376, 512, SWIGLU_UP), 160, gemm_rows.CUT),
+    ((300, 512, 4608, SWIGLU_UP), 160, gemm_rows.CUT),
+    ((300, 512, 17408, SWIGLU_UP), 128, gemm_rows.WHOLE),
+    ((64, 512, 33280, SWIGLU_UP), 256, gemm_rows.TAIL),
+    ((1292, 640, 22980, GELU_UP), 256, gemm_rows.TAIL),
+]
+
+
+def test_gemm_sizes_of_the_operator_tests():
+    made = calls_made([gemm(*size) for size, _, _ in OPS_SIZES])
+    for (size, rows, form), (ok, error, launches) in zip(OPS_SIZES, made):
+        want = gemm_kernels(rows, form, size[3])
+        assert ok, error
+        assert [l.kernel for l in launches][:len(want)] == want, size
