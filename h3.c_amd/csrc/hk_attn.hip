@@ -786,29 +786,60 @@ static float hk_attn_estimate(bool four, uint32_t units, uint32_t tiles,
            rounds(cut, per) + 4.2f + 0.041f * (float)cut;
 }
 
+/* The pieces (1-8) that fill the rounds best: the least rounds of pieces per
+ * piece of an item; 1 where none saves 40% of a round. */
+static uint32_t hk_attn_even_pieces(uint32_t tail, uint32_t tiles,
+                                    uint32_t slots) {
+    uint32_t pieces = 1;
+    float best = 1.0f;
+    for (uint32_t s = 2; tail && s <= 8 && tiles >= 2 * s; s++) {
+        const float cost =
+            (float)((tail * s + slots - 1) / slots) / (float)s;
+        if (cost < best - 1e-6f) {
+            best = cost;
+            pieces = s;
+        }
+    }
+    return best > 0.6f ? 1 : pieces;
+}
+
 /* The fastest of 256-query items, whole or with the last round cut into 2-8
  * pieces, and 128-query items (two a CU, never cut).  Measured at 56 heads
  * (us, whole 256 / best cut / 128): 300 rows 13.7 / 23.4 / 10.9 (cutting
  * any sparse round, as this did, cost 24 us there), 1100 rows 58 / 56 / 41
  * (504 items fit the 512 slots), 1700 rows 97 / 114 / 103, 2378 rows 200 /
  * 178 / 188, 2700 rows 228 / 220 / 215; at 16 heads 1536 rows take 32 with
- * 128-query items, 58 cut into 8.  One round that uses over half the
- * CUs stays whole at 256 queries, where 128 gain nothing (600 rows: 21.3
- * against 22.5). */
+ * 128-query items, 58 cut into 8.
+ * One round that uses over half the CUs stays at 256 queries, where 128 gain
+ * nothing (600 rows x 56 heads: 21.3 against 22.5), and is cut where the
+ * estimate, which takes whole items for up to 15% slower than they are there,
+ * gains over 10%: few heads and long sequences (us, whole and cut, 59 sizes
+ * timed in turn: 1 head x 33240 rows 729 and 551 in 7 pieces, 3 x 11224 248
+ * and 213, 5 x 8408 190 and 182 in 3; below the 10% 3 x 15320 347 and 342, 8 x
+ * 5080 116 and 117, 10 x 4056 94 and 100).
+ * Under half a round, the count that fills the rounds best has 3% in its
+ * favour: the estimate does not see what uneven pieces cost (10 heads x 1280
+ * rows 28.8 us in 4 pieces, 26.8 in 5; 8 x 1900 35.3 in 3, 32.9 in 4). */
 static hk_attn_plan hk_attn_plan_of(uint32_t q_rows, uint32_t kv_rows,
                                     uint32_t heads, uint32_t cus) {
     const uint32_t tiles = (kv_rows + HK_KT - 1) / HK_KT;
     const uint32_t units = (q_rows + HK_QB - 1) / HK_QB * heads;
+    const bool one_round = units <= cus && units * 2 > cus;
     hk_attn_plan plan = {false, 1};
-    if (units <= cus && units * 2 > cus) return plan;
     float best = hk_attn_estimate(false, units, tiles, cus, 1);
+    if (one_round) best *= 0.9f;
+    const uint32_t even = units * 2 <= cus
+                              ? hk_attn_even_pieces(units, tiles, cus)
+                              : 1;
     for (uint32_t s = 2; s <= 8 && tiles >= 2 * s; s++) {
-        const float us = hk_attn_estimate(false, units, tiles, cus, s);
+        float us = hk_attn_estimate(false, units, tiles, cus, s);
+        if (s == even) us *= 0.97f;
         if (us < best) {
             best = us;
             plan.pieces = s;
         }
     }
+    if (one_round) return plan;
     const float narrow = hk_attn_estimate(
         true, (q_rows + 127u) / 128u * heads, tiles, 2 * cus, 1);
     if (1.02f * narrow < best) return {true, 1};
@@ -928,19 +959,10 @@ int hk_attention_bf16(struct h3_gpu *gpu, const uint16_t *q,
         const uint32_t cus = num_cus * (four ? 2u : (uint32_t)HK_WG_PER_CU);
         const uint32_t kv_tiles = (kv_rows + HK_KT - 1) / HK_KT;
         const uint32_t tail = units % cus;
-        uint32_t pieces = four || !tail ? 1 : plan.pieces;
-        if (masked) {
-            float best = 1.0f;
-            for (uint32_t s = 2; tail && s <= 8 && kv_tiles >= 2 * s; s++) {
-                const float cost =
-                    (float)((tail * s + cus - 1) / cus) / (float)s;
-                if (cost < best - 1e-6f) {
-                    best = cost;
-                    pieces = s;
-                }
-            }
-            if (best > 0.6f) pieces = 1;
-        }
+        uint32_t pieces = masked         ? hk_attn_even_pieces(tail, kv_tiles,
+                                                               cus)
+                          : four || !tail ? 1
+                                          : plan.pieces;
         /* scratch: the packed RoPE table, the rotated keys, then the split
          * pieces' partials */
         const size_t table_bytes = ((size_t)a.rope_bytes + 255) & ~(size_t)255;

@@ -26,14 +26,21 @@ def _heads_close(got, q, k, v, rows, heads):
                                                      SCALE))
 
 
-@pytest.mark.parametrize("rows,heads", [
-    (65, 40), (300, 56), (512, 56),  # 128-query items, under a round
-    (600, 56),                       # one round of 256-query items
-    (1100, 56), (2100, 40),          # 128-query items: 504, 680
-    (1200, 56),                      # a cut last round
-    (1700, 56),                      # whole 256-query items, two rounds
-])
-def test_sdpa_plans(gpu, rows, heads):
+# rows, heads, and the plan (test_routes.py checks it): queries an item, pieces
+# of the last round's items
+PLANS = [
+    (65, 40, 128, 1), (300, 56, 128, 1), (512, 56, 128, 1),  # under a round
+    (600, 56, 256, 1),                       # one round, whole
+    (5600, 6, 256, 3), (11224, 3, 256, 5),   # one round, long: cut
+    (1100, 56, 128, 1), (2100, 40, 128, 1),  # 128-query items: 504, 680
+    (1200, 56, 256, 5),                      # a cut last round
+    (1700, 56, 256, 1),                      # two rounds, whole
+    (1280, 10, 256, 5),                      # half a round, even pieces
+]
+
+
+@pytest.mark.parametrize("rows,heads,queries,pieces", PLANS)
+def test_sdpa_plans(gpu, rows, heads, queries, pieces):
     rng = np.random.default_rng(rows + heads)
     q, k, v = (rand_bf16(rng, rows * heads * HD) for _ in range(3))
     out = gpu.new_bf16(rows * heads * HD)

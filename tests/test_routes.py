@@ -1,6 +1,7 @@
 """Which kernels a call launches, on 256 CUs, without a GPU (launches.py)."""
 import pytest
 
+import test_attn_plan_gpu as attn_plan
 import test_gemm_rows_gpu as gemm_rows
 from launches import calls_made
 
@@ -248,3 +249,32 @@ def test_gemm_sizes_of_the_operator_tests():
         want = gemm_kernels(rows, form, size[3])
         assert ok, error
         assert [l.kernel for l in launches][:len(want)] == want, size
+
+
+# measured both ways (us, whole and cut): 33240 x 1 729 and 551, 8408 x 4 185
+# and 165; 8 x 5080 116 and 117, 10 x 4056 94 and 100 stay whole
+PLANS = attn_plan.PLANS + [
+    (33240, 1, 256, 7), (8408, 4, 256, 3), (5080, 8, 256, 1),
+    (4056, 10, 256, 1), (2378, 16, 256, 1), (2378, 56, 256, 5),
+    (2378, 4, 256, 6), (1900, 8, 256, 4), (6144, 40, 256, 1),
+]
+
+
+def test_attention_plans():
+    """How dense attention runs: queries an item, pieces of the last round."""
+    made = calls_made([attention(rows, heads) for rows, heads, _, _ in PLANS])
+    got = []
+    for (rows, heads, _, _), (ok, error, launches) in zip(PLANS, made):
+        assert ok, error
+        names = [l.kernel for l in launches]
+        items = -(-rows // 256) * heads
+        if names == ["hk_flash_fwd<false, false, 4>"]:
+            got.append((rows, heads, 128, 1))
+        elif names == ["hk_flash_fwd<false, false, 8>"]:
+            got.append((rows, heads, 256, 1))
+        else:
+            assert names[-2:] == ["hk_flash_fwd<false, true, 8>",
+                                  "hk_flash_combine<256u>"]
+            got.append((rows, heads, 256,
+                        launches[-2].grid[0] // (items % 256)))
+    assert got == PLANS
