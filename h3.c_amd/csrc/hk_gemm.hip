@@ -315,10 +315,11 @@ extern "C" int h3_hip_gemm_trace_read(uint64_t *out, size_t entries) {
  *
  * XA = 3 hides X's L2 latency behind two steps: with one stage ahead every
  * step waited for it where a CU has only one or two workgroups (40 rows x
- * 5376 -> 21504, 168 workgroups: 46.7 us against 52.8).  With three rounds of
- * workgroups and 33 to 64 rows, XA = 1 is 1.5% ahead (39 rows x 2688 ->
- * 96768: 89.1 us against 90.5 in one run): its smaller LDS lets more
- * workgroups share a CU.
+ * 5376 -> 21504, 168 workgroups: 46.7 us against 52.8).  With several rounds
+ * of workgroups, 33 to 64 rows and K from 1024 on, XA = 1 is level or up to 2%
+ * ahead (64 rows x 2688 -> 96768: 89.6 us against 91.4): its smaller LDS lets
+ * more workgroups share a CU.  With up to 32 rows and a shorter K it is behind
+ * (8 x 2688 -> 96768 78.1 and 75.9; 40 x 320 18.8 and 16.1).
  *
  * Where one workgroup per 128 columns leaves CUs idle, K is split into as
  * many pieces as there are CUs for (blockIdx.y), which write F32 sums that
@@ -419,8 +420,8 @@ hk_gemm_skinny(hk_skinny_args g) {
      * cross. */
     auto in_order = [] { __builtin_amdgcn_sched_barrier(0); };
     /* Steps past the end load zeros (lane offsets beyond the buffers, no
-     * memory touched) and add nothing, so the loop has no branch: behind one,
-     * the compiler drains every load in flight. */
+     * memory touched), so a turn of the ring has no branch: behind one, the
+     * compiler drains every load in flight. */
 #pragma unroll
     for (uint32_t d = 0; d + 1 < D; d++) {
         if (d < XA) stage_x(d, d);
@@ -428,7 +429,38 @@ hk_gemm_skinny(hk_skinny_args g) {
         load_w(d, d);
         in_order();
     }
-    for (uint32_t s0 = 0; s0 < steps; s0 += D) {
+    /* the barrier as inline assembly: __syncthreads() would also wait for
+     * every load in flight (vmcnt(0)), the loads of the steps ahead
+     * included */
+    auto barrier = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    /* W of ring slot d: its lines into the wave's buffer and back out as
+     * fragments (a wave's LDS operations run in order: no barrier), times X
+     * of stage d % (XA + 1) */
+    auto compute = [&](int d) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t r = 8u * q + (lane >> 3);
+            *(hk_v4i *)(wbuf + r * 128u +
+                        (((lane & 7u) ^ hk_swz_key(r)) << 4)) = wf[d][q];
+        }
+        hk_v4i wfrag[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            wfrag[q] = *(const hk_v4i *)(
+                wbuf + row * 128u +
+                (((2u * q + half) ^ hk_swz_key(row)) << 4));
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+                acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(hk_bf16x8, wfrag[q]),
+                    read_x(d % (XA + 1), mb, q), acc[mb], 0, 0, 0);
+    };
+    uint32_t s0 = 0;
+    for (; XA == 1 ? s0 < steps : s0 + D <= steps; s0 += D) {
 #pragma unroll
         for (int d = 0; d < D; d++) {
             const uint32_t s = s0 + d;
@@ -437,37 +469,28 @@ hk_gemm_skinny(hk_skinny_args g) {
             asm volatile("s_waitcnt vmcnt(%0)" ::"i"(
                              4 + (XA - 1) * (MB + 4))
                          : "memory");
-            /* the barrier as inline assembly: __syncthreads() would also
-             * wait for every load in flight (vmcnt(0)), the loads of the
-             * steps ahead included */
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            barrier();
             stage_x((d + XA) % (XA + 1), s + XA);
             in_order();
             load_w((d + 3) % D, s + 3);
-            /* W(s)'s lines into the wave's buffer and back out as
-             * fragments (a wave's LDS operations run in order: no
-             * barrier) */
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint32_t r = 8u * q + (lane >> 3);
-                *(hk_v4i *)(wbuf + r * 128u +
-                            (((lane & 7u) ^ hk_swz_key(r)) << 4)) = wf[d][q];
-            }
-            hk_v4i wfrag[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                wfrag[q] = *(const hk_v4i *)(
-                    wbuf + row * 128u +
-                    (((2u * q + half) ^ hk_swz_key(row)) << 4));
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++)
-                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(hk_bf16x8, wfrag[q]),
-                        read_x(d % (XA + 1), mb, q), acc[mb], 0, 0, 0);
+            compute(d);
         }
     }
+    /* The steps of a last, partial turn, all of them on their way: run as a
+     * whole turn, K = 64 took 4.7 us against 3.9 (32 rows -> 5376 columns).
+     * With XA = 1 it stays a whole turn, whose dead steps add nothing: as
+     * here it took 60 registers more. */
+#pragma unroll
+    for (int d = 0; XA > 1 && d + 1 < D; d++) {
+        if (s0 + d >= steps) break;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(
+                         4 + (XA - 1 - d) * (MB + 4))
+                     : "memory");
+        barrier();
+        compute(d);
+    }
+    /* no load to LDS outlives the workgroup */
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     /* acc[mb][r] = C[mb*32 + row][n0 + (r/4)*8 + half*4 + r%4] */
     if (g.partial) {
         /* whole lines: each (mb, q) is a wave's 64 16-byte pieces */
@@ -865,28 +888,21 @@ static void hk_skinny_lds_setup(const struct h3_gpu *gpu) {
     ready |= bit;
 }
 
-/* Launches hk_gemm_skinny: `problems` of them from a table, or one.  The
- * pieces' sums, at most 64 KiB a CU, go to the context's scratch, which has
- * room for them from its creation: a call that may not allocate finds it
- * there, and calls of two contexts share nothing. */
-static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
-                              const uint16_t *w, const uint16_t *bias,
-                              uint16_t *c, uint32_t m, uint32_t n, uint32_t k,
-                              const uint64_t *group, uint32_t problems,
-                              bool may_allocate) {
-    const uint32_t mbs = (m + 31u) / 32u, wgs = (n + 127u) / 128u;
-    const uint32_t k_steps = k / HK_BK;
-    hk_skinny_args g;
-    g.x = x; g.w = w; g.bias = bias; g.c = c;
-    g.m = m; g.n = n; g.k = k;
-    g.x_bytes = (uint32_t)((uint64_t)m * k * 2);
-    g.w_bytes = (uint32_t)((uint64_t)n * k * 2);
-    g.partial = NULL;
+/* Launches hk_gemm_skinny on the problem(s) of g (X, W, bias, C, their sizes,
+ * group): `problems` from a table, or one.  The pieces' sums, at most 64 KiB a
+ * CU, go to the context's scratch, which has room for them from its creation:
+ * a call that may not allocate finds it there, and calls of two contexts share
+ * nothing. */
+static int hk_gemm_skinny_run(struct h3_gpu *gpu, hk_skinny_args &g,
+                              uint32_t problems, bool may_allocate) {
+    const uint32_t mbs = (g.m + 31u) / 32u, wgs = (g.n + 127u) / 128u;
+    const uint32_t k_steps = g.k / HK_BK;
+    g.x_bytes = (uint32_t)((uint64_t)g.m * g.k * 2);
+    g.w_bytes = (uint32_t)((uint64_t)g.n * g.k * 2);
     g.split_steps = k_steps;
-    g.group = group;
     const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
     /* one workgroup per CU, pieces of at least two turns of the ring */
-    uint32_t splits = group ? 1u : min(cus / wgs, k_steps / 8u);
+    uint32_t splits = g.group ? 1u : min(cus / wgs, k_steps / 8u);
     if (splits > 1) {
         /* whole turns of the kernel's ring of 4 */
         g.split_steps = ((k_steps + splits - 1) / splits + 3u) & ~3u;
@@ -901,18 +917,20 @@ static int hk_gemm_skinny_run(struct h3_gpu *gpu, const uint16_t *x,
         if (!g.partial) splits = 1; /* no scratch: in one piece */
     }
     const dim3 grid(wgs, splits > 1 ? splits : 1u, problems);
-    /* several rounds of few rows: one X stage ahead (both timed above) */
-    const int ahead = mbs <= 2 && wgs * problems >= 2 * cus ? 1 : 3;
-    const size_t lds = mbs * 4096 * (ahead + 1) + 16384;
+    /* one X stage ahead: several rounds of 33 to 64 rows and a long K (both
+     * timed above) */
+    const bool near = mbs == 2 && wgs * problems >= 2 * cus && k_steps >= 16;
+    const size_t lds = mbs * 4096 * (near ? 2 : 4) + 16384;
     void (*kernel)(hk_skinny_args) =
-        mbs == 1   ? (ahead == 1 ? hk_gemm_skinny<1, 1> : hk_gemm_skinny<1, 3>)
-        : mbs == 2 ? (ahead == 1 ? hk_gemm_skinny<2, 1> : hk_gemm_skinny<2, 3>)
+        mbs == 1   ? hk_gemm_skinny<1, 3>
+        : mbs == 2 ? (near ? hk_gemm_skinny<2, 1> : hk_gemm_skinny<2, 3>)
         : mbs == 3 ? hk_gemm_skinny<3, 3>
                    : hk_gemm_skinny<4, 3>;
     if (mbs == 4) hk_skinny_lds_setup(gpu);
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, gpu->stream, g);
     if (g.partial)
-        hipLaunchKernelGGL(hk_skinny_reduce, dim3((n + 31) / 32 * mbs),
+        hipLaunchKernelGGL(hk_skinny_reduce,
+                           dim3((g.n + 31) / 32 * mbs),
                            dim3(256), 0, gpu->stream, g, mbs, wgs * 4,
                            splits);
     return 1;
@@ -926,9 +944,12 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
     const uint64_t w_rows = epilogue == HK_EPI_SWIGLU ? 2ull * n : n;
     const uint64_t x_bytes = (uint64_t)m * k * 2, w_bytes = w_rows * k * 2;
     const bool mfma = hk_gemm_mfma_ok(gpu, x, w, bias, c, m, n, k, epilogue);
-    if (mfma && epilogue == HK_EPI_STORE && m <= HK_SKINNY_ROWS)
-        return hk_gemm_skinny_run(gpu, x, w, bias, c, m, n, k, NULL, 1,
-                                  scratch == NULL);
+    if (mfma && epilogue == HK_EPI_STORE && m <= HK_SKINNY_ROWS) {
+        hk_skinny_args g = {};
+        g.x = x; g.w = w; g.bias = bias; g.c = c;
+        g.m = m; g.n = n; g.k = k;
+        return hk_gemm_skinny_run(gpu, g, 1, scratch == NULL);
+    }
     if (mfma) {
         hk_gemm_lds_setup(gpu);
         hk_gemm_args g;
@@ -1092,11 +1113,14 @@ static int hk_gemm_bf16_group(struct h3_gpu *gpu, const uint16_t *x,
     if (!m || !n || !count) return 1;
     if (m <= HK_SKINNY_ROWS) {
         /* a grid's z dimension ends at 65535 */
-        for (uint32_t p = 0; p < count; p += 65535u)
-            if (!hk_gemm_skinny_run(gpu, x, NULL, NULL, NULL, m, n, k,
-                                    table + (size_t)p * 3,
-                                    min(count - p, 65535u), true))
+        for (uint32_t p = 0; p < count; p += 65535u) {
+            hk_skinny_args g = {};
+            g.x = x;
+            g.m = m; g.n = n; g.k = k;
+            g.group = table + (size_t)p * 3;
+            if (!hk_gemm_skinny_run(gpu, g, min(count - p, 65535u), true))
                 return 0;
+        }
         return 1;
     }
     hk_gemm_lds_setup(gpu);

@@ -99,24 +99,31 @@ def test_gemm_k_loop_has_no_accumulator_copies_or_scratch(extra):
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-@pytest.mark.parametrize("mb,ahead", [(1, 1), (1, 3), (2, 1), (2, 3), (3, 3),
-                                      (4, 3)])
+@pytest.mark.parametrize("mb,ahead", [(1, 3), (2, 1), (2, 3), (3, 3), (4, 3)])
 def test_skinny_loads_leave_in_the_order_its_waits_count(mb, ahead):
     """hk_gemm_skinny<MB, XA> waits until all but the last 4 + (XA - 1)(MB + 4)
     loads have landed, which is X of the step at hand only if every step's MB
-    X loads (to LDS) leave before its four W loads, and steps in order."""
+    X loads (to LDS) leave before its four W loads, and steps in order.  The
+    three steps of a partial turn (none with one stage ahead) load nothing, and
+    nothing is in flight at the end."""
     body = _body(_assembly(),
                  f"_Z14hk_gemm_skinnyILi{mb}ELi{ahead}EEv14hk_skinny_args")
-    loads = "".join("X" if re.search(r"\blds\b", l) else "W"
-                    for l in body if "buffer_load_" in l)
+    loads = [(i, "X" if re.search(r"\blds\b", l) else "W")
+             for i, l in enumerate(body) if "buffer_load_" in l]
     step = "X" * mb + "WWWW"
     ring = "".join("X" * mb * (d < ahead) + "WWWW" for d in range(3))
-    assert loads == ring + 4 * step
+    assert "".join(w for _, w in loads) == ring + 4 * step
     mfma = [i for i, l in enumerate(body) if "v_mfma_" in l]
-    assert len(mfma) == 4 * 4 * mb
-    loop = body[mfma[0]:mfma[-1]]
-    assert not [l for l in loop if "s_cbranch" in l or "scratch_" in l]
+    assert len(mfma) == (4 + 3 * (ahead > 1)) * 4 * mb
+    # the turn comes first, its loads (but the first X) among its MFMAs
+    first, last = mfma[0], mfma[4 * 4 * mb - 1]
+    among = "".join(w for i, w in loads if first < i < last)
+    assert (4 * step).endswith(among) and among.endswith(3 * step)
+    assert not [l for l in body[first:last]
+                if "s_cbranch" in l or "scratch_" in l]
     # the kernel's own waits, apart from the compiler's
     asm = re.findall(r"#ASMSTART\n\s*s_waitcnt vmcnt\((\d+)\)",
                      "\n".join(body))
-    assert asm == [str(4 + (ahead - 1) * (mb + 4))] * 4
+    turn = [4 + (ahead - 1) * (mb + 4)] * 4
+    tail = [4 + (2 - d) * (mb + 4) for d in range(3)] if ahead > 1 else []
+    assert [int(w) for w in asm] == turn + tail + [0]

@@ -148,6 +148,17 @@ def test_few_rows_take_the_skinny_kernel_with_any_weight(rows, kernel):
         assert launches[0].kernel in (kernel, kernel[:-2] + "3>")
 
 
+def test_one_x_stage_ahead_for_rounds_of_two_row_blocks_and_long_k():
+    sizes = {(40, 2688, 96768): "hk_gemm_skinny<2, 1>",
+             (40, 320, 96768): "hk_gemm_skinny<2, 3>",
+             (64, 1024, 32768): "hk_gemm_skinny<2, 3>",
+             (8, 2688, 96768): "hk_gemm_skinny<1, 3>"}
+    made = calls_made([linear(*size) for size in sizes])
+    for (ok, error, launches), kernel in zip(made, sizes.values()):
+        assert ok, error
+        assert [l.kernel for l in launches] == [kernel]
+
+
 STORE, SWIGLU_UP, GELU_UP = 0, 1, 2
 
 

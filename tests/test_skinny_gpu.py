@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
     (65, 64, 128, True), (96, 128, 132, False),   # 3 row blocks, 1-2 K steps
     (97, 320, 100, True), (128, 448, 4, True),    # 4 row blocks, K steps 5, 7
     (129, 512, 260, True),                        # one past: the tile kernel
-    (1, 64, 4, True), (1, 192, 4, False),         # dead steps pass both ends
+    (1, 64, 4, True), (1, 192, 4, False),         # a partial turn of the ring
+    (33, 128, 300, True), (128, 192, 260, False),
+    (40, 384, 260, True), (64, 1088, 65540, False),  # 6 steps; 17, one ahead
     (1, 1024, 4, True), (7, 2112, 36, False),     # split K, a short last piece
     (33, 4096, 300, True), (120, 5120, 1284, True),
     (128, 14336, 128, False),                     # 28 pieces of one tile
