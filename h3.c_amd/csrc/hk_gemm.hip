@@ -344,6 +344,10 @@ struct hk_skinny_args {
     uint32_t split_steps;
     /* problem blockIdx.z's W, bias and C (a grouped launch), or null */
     const uint64_t *group;
+    /* problem 1's W, bias and C of a paired launch (w1 null: one problem);
+     * its pieces' sums follow those of problem 0 */
+    const uint16_t *w1, *bias1;
+    uint16_t *c1;
 };
 
 template <int MB, int XA>
@@ -356,6 +360,10 @@ hk_gemm_skinny(hk_skinny_args g) {
         w = (const uint16_t *)hk_group_word(g.group, 3 * blockIdx.z);
         bias = (const uint16_t *)hk_group_word(g.group, 3 * blockIdx.z + 1);
         c = (uint16_t *)hk_group_word(g.group, 3 * blockIdx.z + 2);
+    } else if (blockIdx.z) {
+        w = g.w1;
+        bias = g.bias1;
+        c = g.c1;
     }
     /* k steps of this split; its byte offset goes in the scalar offsets */
     const uint32_t base = g.partial ? blockIdx.y * g.split_steps : 0u;
@@ -496,7 +504,8 @@ hk_gemm_skinny(hk_skinny_args g) {
         /* whole lines: each (mb, q) is a wave's 64 16-byte pieces */
         hk_f32x4 *part =
             (hk_f32x4 *)g.partial +
-            ((size_t)blockIdx.y * gridDim.x * 4u + blockIdx.x * 4u + wave) *
+            (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x * 4u +
+             blockIdx.x * 4u + wave) *
                 (MB * 256u);
         if (n0 >= n) return;
 #pragma unroll
@@ -539,25 +548,29 @@ hk_gemm_skinny(hk_skinny_args g) {
 __global__ void __launch_bounds__(256)
 hk_skinny_reduce(hk_skinny_args g, uint32_t mbs, uint32_t tiles,
                  uint32_t splits) {
-    /* blockIdx.x = tile * mbs + mb; threads run over (q, lane) */
+    /* blockIdx.x = tile * mbs + mb, blockIdx.y the problem of a paired
+     * launch; threads run over (q, lane) */
     const uint32_t lane = threadIdx.x & 63u, q = threadIdx.x >> 6;
     const uint32_t tile = blockIdx.x / mbs, mb = blockIdx.x % mbs;
     const uint32_t row = mb * 32u + (lane & 31u);
     const uint32_t col = tile * 32u + q * 8u + (lane >> 5) * 4u;
     if (row >= g.m || col >= g.n) return;
-    const hk_f32x4 *p = (const hk_f32x4 *)g.partial +
-                        (size_t)blockIdx.x * 256u + threadIdx.x;
+    const uint16_t *bias = blockIdx.y ? g.bias1 : g.bias;
+    uint16_t *c = blockIdx.y ? g.c1 : g.c;
     const size_t stride = (size_t)tiles * mbs * 256u;
+    const hk_f32x4 *p = (const hk_f32x4 *)g.partial +
+                        blockIdx.y * splits * stride +
+                        (size_t)blockIdx.x * 256u + threadIdx.x;
     hk_f32x4 sum = *p;
     for (uint32_t s = 1; s < splits; s++) sum += p[s * stride];
-    if (g.bias) {
-        const uint2 b = *(const uint2 *)(g.bias + col);
+    if (bias) {
+        const uint2 b = *(const uint2 *)(bias + col);
         sum[0] += hk_bf2f(b.x & 0xffffu);
         sum[1] += hk_bf2f(b.x >> 16);
         sum[2] += hk_bf2f(b.y & 0xffffu);
         sum[3] += hk_bf2f(b.y >> 16);
     }
-    *(uint2 *)(g.c + (size_t)row * g.n + col) =
+    *(uint2 *)(c + (size_t)row * g.n + col) =
         make_uint2(hk_pack2(sum[0], sum[1]), hk_pack2(sum[2], sum[3]));
 }
 
@@ -889,10 +902,10 @@ static void hk_skinny_lds_setup(const struct h3_gpu *gpu) {
 }
 
 /* Launches hk_gemm_skinny on the problem(s) of g (X, W, bias, C, their sizes,
- * group): `problems` from a table, or one.  The pieces' sums, at most 64 KiB a
- * CU, go to the context's scratch, which has room for them from its creation:
- * a call that may not allocate finds it there, and calls of two contexts share
- * nothing. */
+ * group or w1 ...): `problems` from a table, a pair, or one.  The pieces'
+ * sums, at most 64 KiB a CU, go to the context's scratch, which has room for
+ * them from its creation: a call that may not allocate finds it there, and
+ * calls of two contexts share nothing. */
 static int hk_gemm_skinny_run(struct h3_gpu *gpu, hk_skinny_args &g,
                               uint32_t problems, bool may_allocate) {
     const uint32_t mbs = (g.m + 31u) / 32u, wgs = (g.n + 127u) / 128u;
@@ -902,14 +915,15 @@ static int hk_gemm_skinny_run(struct h3_gpu *gpu, hk_skinny_args &g,
     g.split_steps = k_steps;
     const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
     /* one workgroup per CU, pieces of at least two turns of the ring */
-    uint32_t splits = g.group ? 1u : min(cus / wgs, k_steps / 8u);
+    uint32_t splits =
+        g.group ? 1u : min(cus / (wgs * problems), k_steps / 8u);
     if (splits > 1) {
         /* whole turns of the kernel's ring of 4 */
         g.split_steps = ((k_steps + splits - 1) / splits + 3u) & ~3u;
         splits = (k_steps + g.split_steps - 1) / g.split_steps;
     }
     if (splits > 1) {
-        const size_t bytes = (size_t)splits * wgs * 4 * mbs * 4096;
+        const size_t bytes = (size_t)problems * splits * wgs * 4 * mbs * 4096;
         if (may_allocate)
             g.partial = (float *)hk_splitk_try(gpu, bytes);
         else if (bytes <= gpu->splitk_bytes)
@@ -930,9 +944,8 @@ static int hk_gemm_skinny_run(struct h3_gpu *gpu, hk_skinny_args &g,
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, gpu->stream, g);
     if (g.partial)
         hipLaunchKernelGGL(hk_skinny_reduce,
-                           dim3((g.n + 31) / 32 * mbs),
-                           dim3(256), 0, gpu->stream, g, mbs, wgs * 4,
-                           splits);
+                           dim3((g.n + 31) / 32 * mbs, problems), dim3(256), 0,
+                           gpu->stream, g, mbs, wgs * 4, splits);
     return 1;
 }
 
@@ -1064,11 +1077,18 @@ int hk_gemm_bf16_pair(struct h3_gpu *gpu, const uint16_t *x,
     const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
     const uint32_t tiles = ((m + HK_BM - 1) / HK_BM) * ((n + HK_BN - 1) / HK_BN);
     const uint32_t k_steps = k / HK_BK;
-    const bool paired =
-        m > HK_SKINNY_ROWS && k_steps >= 8 && tiles * 4 <= cus &&
+    const bool mfma =
         hk_gemm_mfma_ok(gpu, x, w0, b0, c0, m, n, k, HK_EPI_STORE) &&
         hk_gemm_mfma_ok(gpu, x, w1, b1, c1, m, n, k, HK_EPI_STORE);
-    if (!paired)
+    /* few rows: one skinny launch while a round of CUs holds both */
+    if (mfma && m <= HK_SKINNY_ROWS && (n + 127u) / 128u * 2 <= cus) {
+        hk_skinny_args g = {};
+        g.x = x; g.w = w0; g.bias = b0; g.c = c0;
+        g.m = m; g.n = n; g.k = k;
+        g.w1 = w1; g.bias1 = b1; g.c1 = c1;
+        return hk_gemm_skinny_run(gpu, g, 2, true);
+    }
+    if (!mfma || m <= HK_SKINNY_ROWS || k_steps < 8 || tiles * 4 > cus)
         return hk_gemm_bf16(gpu, x, w0, b0, c0, m, n, k, HK_EPI_STORE) &&
                hk_gemm_bf16(gpu, x, w1, b1, c1, m, n, k, HK_EPI_STORE);
     hk_gemm_lds_setup(gpu);

@@ -212,11 +212,12 @@ int h3_hip_head_rms_norm_group_bf16(h3_gpu *gpu, const h3_gpu_tensor *table,
 
 /* Two projections of one input, output0 = X . weight0^T + bias0 and
  * output1 = X . weight1^T + bias1, each exactly as h3_gpu_linear_bf16
- * computes it (f32 accumulation, one bf16 rounding).  Small launches
- * (over 128 rows and together at most half the CUs' worth of 256x256 tiles,
- * such as the text's cross-attention K and V) share one split-K launch;
- * others run as two linears.  Biases may be NULL.  No reference counterpart: the
- * reference has no cross-attention. */
+ * computes it (f32 accumulation, one bf16 rounding).  Small launches (up to
+ * 128 rows: together at most one 128-column workgroup a CU; over 128: together
+ * at most half the CUs' worth of 256x256 tiles, such as the text's
+ * cross-attention K and V) share one split-K launch; others run as two
+ * linears.  Biases may be NULL.  No reference counterpart: the reference has
+ * no cross-attention. */
 int h3_hip_linear_pair_bf16(h3_gpu *gpu, h3_gpu_tensor *output0,
                             h3_gpu_tensor *output1,
                             const h3_gpu_tensor *input,

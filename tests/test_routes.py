@@ -159,6 +159,35 @@ def test_one_x_stage_ahead_for_rounds_of_two_row_blocks_and_long_k():
         assert [l.kernel for l in launches] == [kernel]
 
 
+def pair(m, k, n):
+    return ["h3_hip_linear_pair_bf16", *[["bf16", m * n]] * 2,
+            ["bf16", m * k], ["bf16", n * k], ["bf16", n], ["bf16", n * k],
+            None, m, k, n]
+
+
+@pytest.mark.parametrize("limit", [None, 0])
+def test_a_pair_of_few_rows_is_one_launch(limit):
+    """Both problems in one skinny launch (grid z) and one sum of the pieces,
+    within the scratch that the context holds; in two past one round of CUs."""
+    sizes = [(1, 64, 4), (65, 512, 132), (128, 14336, 128), (97, 5120, 5120),
+             (40, 128, 16384), (40, 128, 16388)]
+    made = calls_made([pair(*size) for size in sizes], largest_block=limit)
+    for (m, k, n), (ok, error, launches) in zip(sizes, made):
+        assert ok and not error, error
+        kernel = f"hk_gemm_skinny<{(m + 31) // 32}, 3>"
+        wgs = -(-n // 128)
+        if 2 * wgs > 256:
+            assert [l.kernel for l in launches] == [kernel, kernel]
+            continue
+        first, *rest = launches
+        assert first.kernel == kernel and first.grid[2] == 2
+        assert 2 * wgs * first.grid[1] <= 256
+        cut = first.grid[1] > 1
+        assert cut == (k >= 1024)
+        assert [(l.kernel, l.grid[1]) for l in rest] == (
+            [("hk_skinny_reduce", 2)] if cut else [])
+
+
 STORE, SWIGLU_UP, GELU_UP = 0, 1, 2
 
 

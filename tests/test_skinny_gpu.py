@@ -38,6 +38,26 @@ def test_linear_skinny(gpu, m, k, n, bias):
     assert np.array_equal(gpu.read_bf16(out), got)
 
 
+@pytest.mark.parametrize("m,k,n", [
+    (1, 64, 4), (65, 512, 132), (97, 1088, 260),
+    (8, 5376, 512), (128, 14336, 128),  # K in pieces
+    (40, 128, 16384), (40, 128, 16388),  # the last size in one launch, and two
+])
+def test_linear_pair_skinny(gpu, m, k, n):
+    """Each of a pair is what a linear gives (its sums in other pieces where K
+    is cut)."""
+    rng = np.random.default_rng(m + k + n)
+    x = rand_bf16(rng, m * k)
+    ws = [rand_bf16(rng, n * k, 0.05) for _ in range(2)]
+    bs = [rand_bf16(rng, n, 0.1), None]
+    outs = [gpu.new_bf16(m * n) for _ in range(2)]
+    gpu.run("h3_hip_linear_pair_bf16", *outs, gpu.bf16(x), gpu.bf16(ws[0]),
+            gpu.bf16(bs[0]), gpu.bf16(ws[1]), None, m, k, n)
+    for out, w, b in zip(outs, ws, bs):
+        assert_close(gpu.read_bf16(out), oracle.linear(x, w, b, m, k, n),
+                     what="skinny pair")
+
+
 @pytest.mark.parametrize("m,k,n,count,first", [
     (1, 64, 64, 3, 0), (40, 320, 132, 4, 1), (64, 512, 640, 5, 2),
     (65, 128, 128, 2, 0), (120, 512, 260, 3, 1),
