@@ -890,6 +890,21 @@ static uint32_t hk_gemm_row_blocks(uint32_t m, uint32_t columns,
     return best;
 }
 
+/* Whether the skinny kernel takes a plain linear: up to 128 rows, but not 97
+ * to 128 of a short K where its 128-column workgroups, each on half a CU,
+ * fill one to two CU rounds unevenly and the tiles, twice as wide, at most
+ * one (128 rows, us skinny and tiles: 64 -> 60000 columns 11.6 and 10.9, 320
+ * -> 52000 17.7 and 14.7, 512 -> 36000 20.7 and 16.0; a longer K gains up to
+ * half that width and loses beyond, 1024 -> 36000 29.8 and 25.7, -> 60000
+ * 32.4 and 35.6).  Those tiles are never cut, so a call that may not
+ * allocate needs no scratch. */
+static bool hk_skinny_takes(uint32_t m, uint32_t n, uint32_t k,
+                            uint32_t cus) {
+    const uint32_t wgs = (n + 127u) / 128u;
+    return m <= HK_SKINNY_ROWS &&
+           !(m > 96 && k <= 512 && wgs > cus && wgs <= 2 * cus);
+}
+
 /* 80 KiB of dynamic LDS need the kernel's limit raised, once per device. */
 static void hk_skinny_lds_setup(const struct h3_gpu *gpu) {
     static uint64_t ready = 0;
@@ -957,7 +972,8 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
     const uint64_t w_rows = epilogue == HK_EPI_SWIGLU ? 2ull * n : n;
     const uint64_t x_bytes = (uint64_t)m * k * 2, w_bytes = w_rows * k * 2;
     const bool mfma = hk_gemm_mfma_ok(gpu, x, w, bias, c, m, n, k, epilogue);
-    if (mfma && epilogue == HK_EPI_STORE && m <= HK_SKINNY_ROWS) {
+    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
+    if (mfma && epilogue == HK_EPI_STORE && hk_skinny_takes(m, n, k, cus)) {
         hk_skinny_args g = {};
         g.x = x; g.w = w; g.bias = bias; g.c = c;
         g.m = m; g.n = n; g.k = k;
@@ -968,7 +984,6 @@ int hk_gemm_bf16(struct h3_gpu *gpu, const uint16_t *x, const uint16_t *w,
         hk_gemm_args g;
         g.x = x; g.w = w; g.bias = bias; g.c = c;
         g.m = m; g.n = n; g.k = k;
-        const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
         const uint32_t cols_per_tile = epilogue == HK_EPI_SWIGLU ? 128 : HK_BN;
         const uint32_t k_steps = k / HK_BK;
         g.tiles_n = (n + cols_per_tile - 1) / cols_per_tile;

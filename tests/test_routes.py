@@ -159,6 +159,24 @@ def test_one_x_stage_ahead_for_rounds_of_two_row_blocks_and_long_k():
         assert [l.kernel for l in launches] == [kernel]
 
 
+def test_up_to_128_rows_between_one_and_two_rounds():
+    """97 to 128 rows of a short K whose skinny workgroups would fill between
+    one and two rounds take tiles, never cut (no scratch in a call that may
+    not allocate, whose contexts may overlap)."""
+    tiles = [(97, 64, 36000), (128, 512, 32772), (128, 320, 65536),
+             (100, 512, 45000)]
+    skinny = [(96, 512, 36000), (128, 512, 32768), (128, 512, 65540),
+              (128, 576, 36000), (1, 64, 36000)]
+    made = calls_made([linear(*size, "h3_hip_linear_bf16_noalloc")
+                       for size in tiles + skinny], largest_block=0)
+    for i, (ok, error, launches) in enumerate(made):
+        assert ok and not error, error
+        kernel, = [l.kernel for l in launches]
+        assert kernel.startswith("hk_gemm_mfma" if i < len(tiles) else
+                                 "hk_gemm_skinny"), (tiles + skinny)[i]
+        assert kernel.split("<")[1][0] == "0" or i >= len(tiles)
+
+
 def pair(m, k, n):
     return ["h3_hip_linear_pair_bf16", *[["bf16", m * n]] * 2,
             ["bf16", m * k], ["bf16", n * k], ["bf16", n], ["bf16", n * k],

@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
     (65, 64, 128, True), (96, 128, 132, False),   # 3 row blocks, 1-2 K steps
     (97, 320, 100, True), (128, 448, 4, True),    # 4 row blocks, K steps 5, 7
     (129, 512, 260, True),                        # one past: the tile kernel
+    (128, 64, 32772, True), (97, 512, 33000, False),  # tiles, short K and wide
     (1, 64, 4, True), (1, 192, 4, False),         # a partial turn of the ring
     (33, 128, 300, True), (128, 192, 260, False),
     (40, 384, 260, True), (64, 1088, 65540, False),  # 6 steps; 17, one ahead
