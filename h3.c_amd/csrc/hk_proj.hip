@@ -184,6 +184,10 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
         ((uintptr_t)w & 15) || (uint64_t)m * k * 4 + margin >= 0x100000000ull ||
         (uint64_t)n * k * 4 + margin >= 0x100000000ull || m > 65535u * 64u)
         return false;
+    /* a handful of products each: one thread an output is done before eight
+     * waves have met (K = 16, 128 x 64 outputs 3.5 us against 4.6, 128 x 512
+     * 3.5 against 4.8; 300 x 512 7.1 against 4.9) */
+    if (k <= 16 && (uint64_t)m * n <= 65536) return false;
     struct {
         uint32_t blocks;
         void (*kernel)(hk_linear_f32_args);
@@ -196,13 +200,21 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
     /* the fewest row blocks of 16 that hold m, at most 8 a workgroup */
     uint32_t at = 0;
     while (at < 5 && sizes[at].blocks * 16u < m) at++;
+    const uint32_t gx = (n + 16 * HK_LF_BLOCKS - 1) / (16 * HK_LF_BLOCKS);
+    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
+    const uint32_t steps = (k + 31u) / 32u;
+    /* a K too short for pieces: fewer rows a workgroup, from 32 on, while one
+     * round of CUs holds them (128 rows x 64 -> 64 5.0 us against 9.2 with all
+     * rows in one, and 7.4 of one thread an output; 300 x 256 -> 512 6.4
+     * against 11.5; beyond a round 1000 x 128 -> 5376 66 against 56) */
+    for (uint32_t few = 1; few < at && steps < 8 * HK_LF_WAVES; few++)
+        if ((uint64_t)gx * ((m + 16 * sizes[few].blocks - 1) /
+                            (16 * sizes[few].blocks)) <= cus)
+            at = few;
     const uint32_t mb = sizes[at].blocks;
     const uint32_t lds =
         HK_LF_WAVES * HK_LF_BLOCKS * mb * 64 * (uint32_t)sizeof(hk_f32x4);
-    const uint32_t gx = (n + 16 * HK_LF_BLOCKS - 1) / (16 * HK_LF_BLOCKS);
     const uint32_t gy = (m + 16 * mb - 1) / (16 * mb);
-    const uint32_t cus = gpu->num_cus > 0 ? (uint32_t)gpu->num_cus : 256u;
-    const uint32_t steps = (k + 31u) / 32u;
     /* pieces of at least 4 steps a wave, while they find idle CUs */
     uint32_t pieces = gx * gy <= cus ? cus / (gx * gy) : 1u;
     if (pieces > steps / (4 * HK_LF_WAVES)) pieces = steps / (4 * HK_LF_WAVES);
@@ -223,10 +235,14 @@ bool hk_linear_f32(struct h3_gpu *gpu, const float *x, const float *w,
         }
     }
     if (pieces < 1) pieces = 1;
-    if (lds > 64 * 1024)
+    static uint64_t ready[2]; /* devices whose limit is raised: 96, 128 rows */
+    const uint64_t bit = 1ull << (gpu->device & 63);
+    if (lds > 64 * 1024 && !(ready[at - 4] & bit)) {
         (void)hipFuncSetAttribute((const void *)sizes[at].kernel,
                                   hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)lds);
+        ready[at - 4] |= bit;
+    }
     hipLaunchKernelGGL(sizes[at].kernel, dim3(gx, gy, pieces),
                        dim3(HK_LF_WAVES * 64), lds, gpu->stream, g);
     if (pieces > 1)
@@ -357,7 +373,8 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
                      uint32_t k) {
     if (gpu->reference_kernels || !k || k % 4 || n % 4 ||
         ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
-        ((uintptr_t)bias & 15) || ((uintptr_t)out & 7) || m > 65535u * HK_PL_ROWS)
+        ((uintptr_t)bias & 15) || ((uintptr_t)out & 7) ||
+        m > 65535u * HK_PL_ROWS)
         return false;
     hipLaunchKernelGGL(hk_patch_linear_mfma,
                        dim3((n + HK_PL_COLS - 1) / HK_PL_COLS,
@@ -617,7 +634,8 @@ bool hk_adaln_head(struct h3_gpu *gpu, const uint16_t *x, float *inverse,
                    uint32_t shift_slot, uint32_t scale_slot, float epsilon) {
     /* a thread per 8 columns, loaded 16 bytes at a time */
     if (gpu->reference_kernels || width % 32 ||
-        width > HK_HEAD_WAVES * 64 * 8 || !n || n > 65535u * 32u || ((uintptr_t)x & 15) || ((uintptr_t)norm & 15) ||
+        width > HK_HEAD_WAVES * 64 * 8 || !n || n > 65535u * 32u ||
+        ((uintptr_t)x & 15) || ((uintptr_t)norm & 15) ||
         ((uintptr_t)mod & 15) || ((uintptr_t)w & 15))
         return false;
     const hk_head_args a = {x,       norm, mod, w,     bias,  row_map,

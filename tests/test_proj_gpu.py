@@ -12,12 +12,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m,k,n", [
-    (1, 4, 1), (3, 20, 5),          # one step, a step's tail
+    (1, 4, 1), (3, 20, 5),          # one thread an output, a step's tail
     (16, 256, 16), (17, 260, 33),   # a full tile, one row and column more
     (33, 128, 47), (48, 96, 64), (49, 2052, 31),
     (64, 516, 18), (65, 512, 17), (96, 1040, 16), (97, 64, 5),
     (128, 300, 33), (129, 96, 20),  # every height, one and two row blocks
     (39, 256, 5376), (101, 5376, 2688),
+    (65, 2048, 33), (96, 2052, 17),  # 96 rows a workgroup
+    (1000, 128, 512), (128, 64, 5376), (70000, 4, 3),
     (5, 7, 9),                      # K % 4 != 0: the general kernel
 ])
 def test_linear_f32(gpu, m, k, n):

@@ -34,6 +34,28 @@ def linear_f32(m, k, n):
             ["f32", n * k], ["f32", n], m, k, n]
 
 
+# rows, K, N, row blocks of 16 a workgroup; where K has pieces, or one round
+# of CUs does not hold fewer rows a workgroup, the fewest that hold all rows
+LINEAR_F32 = [(39, 256, 5376, 3), (101, 5376, 2688, 8), (39, 5376, 2688, 3),
+              (16, 64, 64, 1), (39, 64, 64, 2), (128, 64, 64, 2),
+              (1000, 128, 64, 2), (1000, 128, 512, 4), (128, 64, 5376, 8),
+              (128, 2016, 64, 2), (128, 2048, 64, 8)]
+
+
+def test_f32_linear_rows_of_a_workgroup():
+    made = calls_made([linear_f32(*size[:3]) for size in LINEAR_F32])
+    for (m, k, n, blocks), (ok, error, launches) in zip(LINEAR_F32, made):
+        assert ok, error
+        kernel = launches[0].kernel
+        assert kernel.startswith(f"hk_linear_f32_mfma<{blocks}, "), (m, k, n)
+        assert launches[0].lds <= max(launches[0].lds_limit, 64 * 1024)
+    # few products each: one thread an output, up to 65536 outputs
+    made = calls_made([linear_f32(128, 16, 512), linear_f32(129, 16, 512),
+                       linear_f32(128, 20, 512)])
+    assert [launches[0].kernel[:18] for _, _, launches in made] == [
+        "hk_linear_f32_kern", "hk_linear_f32_mfma", "hk_linear_f32_mfma"]
+
+
 def patch(rows, k, n):
     return ["h3_hip_patch_linear_bf16_offset", ["bf16", rows * n], 0,
             ["f32", rows * k], 0, ["f32", n * k], ["f32", n], rows, k, n]
