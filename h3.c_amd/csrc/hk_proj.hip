@@ -632,8 +632,14 @@ bool hk_adaln_head(struct h3_gpu *gpu, const uint16_t *x, float *inverse,
                    const uint16_t *bias, uint16_t *out, uint32_t rows,
                    uint32_t width, uint32_t n, uint32_t slots,
                    uint32_t shift_slot, uint32_t scale_slot, float epsilon) {
-    /* a thread per 8 columns, loaded 16 bytes at a time */
+    /* a thread per 8 columns, loaded 16 bytes at a time; of a small weight,
+     * smaller with many rows, one workgroup a row is faster (us at 74, 1792
+     * and 6000 rows, here and there: 64 -> 4 6.8, 10.5 and 19.8, 4.0, 4.1 and
+     * 8.1; 64 -> 64 11.3, 12.5 and 26.3, 9.4, 11.9 and 33.5; 256 -> 32 9.5,
+     * 12.2 and 23.0, 8.5, 10.7 and 27.8; 128 -> 96 11.4, 12.5 and 28.8, 15.5,
+     * 19.4 and 54.4) */
     if (gpu->reference_kernels || width % 32 ||
+        (uint64_t)width * n < (rows <= 2048 ? 12288u : 4096u) ||
         width > HK_HEAD_WAVES * 64 * 8 || !n || n > 65535u * 32u ||
         ((uintptr_t)x & 15) || ((uintptr_t)norm & 15) ||
         ((uintptr_t)mod & 15) || ((uintptr_t)w & 15))

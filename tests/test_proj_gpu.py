@@ -100,8 +100,9 @@ def test_patch_linear_tiles_bit_exact(gpu, rows, k, n, mapped):
     (33, 5376, 32), (3, 512, 97), (2, 8192, 48),
     (1025, 64, 32), (517, 96, 33),  # 16 rows a workgroup
     (2049, 64, 96), (2100, 5376, 50),  # and 96 columns
+    (1, 4096, 3), (1025, 384, 32), (517, 128, 97), (2049, 128, 96),
     (1025, 4032, 32), (1040, 4000, 96),  # just over 64 KiB of LDS
-    (4, 8224, 96), (4, 264, 8),  # the general kernel
+    (4, 8224, 96), (4, 264, 8),  # the general kernel, as with small weights
 ])
 @pytest.mark.parametrize("shared", [True, False])
 def test_adaln_head_tiles(gpu, rows, width, n, shared):

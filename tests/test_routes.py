@@ -29,6 +29,20 @@ def test_head_lds_limit(rows, n, width):
         assert launch.lds_limit > 64 * 1024
 
 
+@pytest.mark.parametrize("rows,width,n,kernel", [
+    (74, 5376, 32, "hk_adaln_head_mfma"), (74, 128, 96, "hk_adaln_head_mfma"),
+    (2048, 352, 32, "hk_adaln_head_kernel"),
+    (2049, 352, 32, "hk_adaln_head_mfma"),
+    (2049, 64, 64, "hk_adaln_head_mfma"),
+    (2049, 64, 63, "hk_adaln_head_kernel"),
+    (74, 32, 383, "hk_adaln_head_kernel"), (74, 32, 384, "hk_adaln_head_mfma"),
+])
+def test_head_of_a_small_weight(rows, width, n, kernel):
+    (ok, error, (launch,)), = calls_made([head(rows, width, n)])
+    assert ok, error
+    assert launch.kernel.split("<")[0] == kernel
+
+
 def linear_f32(m, k, n):
     return ["h3_gpu_linear_f32", ["f32", m * n], ["f32", m * k],
             ["f32", n * k], ["f32", n], m, k, n]
