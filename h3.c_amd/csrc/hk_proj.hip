@@ -398,8 +398,10 @@ bool hk_patch_linear(struct h3_gpu *gpu, const float *x, const float *w,
  * are 168 KiB) to be MFMA operands (v_mfma_f32_16x16x32_bf16), and the waves
  * split the half's 32-wide k steps, reading weight rows from L2.
  *
- * A CU takes 64 bytes a clock from its L1, which bounds this kernel: 0.7 MiB
- * a workgroup with NB = 3 (half of it weights).  Loading x, norm, shift and
+ * What bounds it is a workgroup's one dependent chain: x from memory, the
+ * statistics, two barriers, the normalised rows to LDS, then the weights
+ * (three quarters of the 0.7 MiB that a workgroup reads with NB = 3, which
+ * alone takes 5 us of a CU's 64 bytes a clock).  Loading x, norm, shift and
  * scale as MFMA fragments instead (16 lanes repeating each modulation piece)
  * took 41-44 us at 1792 rows x 96 outputs and 21 us at 74 rows x 32; this
  * takes 24.2 and 15.4 us, with the modulation rows' numbers, the modulation
@@ -428,7 +430,8 @@ hk_adaln_head_mfma(hk_head_args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t hk_head_lds[];
     __shared__ float squares[HK_HEAD_WAVES][ROWS];
     __shared__ float inverses[ROWS];
-    /* weight steps in flight: as many as the registers hold */
+    /* weight steps in flight: as many as the 128 registers hold (of NB = 6
+     * even one spills ten; it is still the faster there, see hk_adaln_head) */
     constexpr uint32_t AHEAD = NB > 3 ? 1 : NB * ROWS > 32 ? 2 : 3;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
