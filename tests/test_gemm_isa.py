@@ -38,6 +38,12 @@ INSTANCES = {
     "hk_gemm_mfma<4> (split-K SwiGLU)":
         "_Z12hk_gemm_mfmaILi4ELb0EEv12hk_gemm_args",
 }
+# the tiles of 128 to 224 rows; nothing cuts 224-row tiles along K
+INSTANCES.update({
+    f"hk_gemm_mfma_low<{epi}, {'group, ' * group}{jb}>":
+        f"_Z16hk_gemm_mfma_lowILi{epi}ELb{group}ELi{jb}EEv12hk_gemm_args"
+    for epi, group in [(0, 0), (1, 0), (2, 0), (0, 1), (3, 0), (4, 0)]
+    for jb in (4, 5, 6, 7) if jb < 7 or epi < 3})
 BAD = re.compile(r"\b(v_accvgpr_mov_b32|v_accvgpr_write_b32|scratch_\w+)\b")
 
 
@@ -70,7 +76,8 @@ def _k_loop_offenders(extra):
     for name, sym in INSTANCES.items():
         body = _body(text, sym)
         mfma = [i for i, l in enumerate(body) if "v_mfma_" in l]
-        assert len(mfma) == 128, (name, len(mfma))
+        jb = int((re.search(r"ELi(\d)EEv", sym) or [8, 8])[1])
+        assert len(mfma) == 16 * jb, (name, len(mfma))
         loop = body[mfma[0]:mfma[-1]]
         found[name] = [l.strip() for l in loop if BAD.search(l)]
         waits = [int(m.group(1)) for l in loop
