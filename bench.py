@@ -277,9 +277,9 @@ def h3_measure(gpu, blocks, reps, latent_h=32, latent_w=32, full=True):
         kern = {}
         for cname, mask, what in (
                 ("gemm_plain", OPS_GEMM, "QKV + out-projection "
-                 "(hk_gemm_mfma<0>, split tails)"),
+                 "(hk_gemm_mfma<0> or _low<0>, tile height by row count)"),
                 ("mlp_swiglu", OPS_ACT, "fc1 with SwiGLU epilogue "
-                 "(hk_gemm_mfma<1>) + fc2 (hk_gemm_mfma<0>)"),
+                 "(hk_gemm_mfma<1> or _low<1>) + fc2 (<0>)"),
                 ("attention", OPS_ATTN, "hk_flash_fwd (joint self-"
                  "attention, key-split last round)"),
                 ("row_ops", OPS_ROWS, "adaLN / gate+adaLN / grouped Q-K "
