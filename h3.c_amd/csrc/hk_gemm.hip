@@ -840,7 +840,9 @@ static float hk_gemm_estimate(uint32_t jb, uint32_t tiles, uint32_t k_steps,
  *   254 us).
  * The gain has to be over 2%, and over 5%, the estimate's error there, if the
  * 256-row tiles end in a cut tail and the lower ones need several bands (6144
- * x 5120 -> 13824: 0.5% by the estimate, 688 and 696 us with 224 rows).
+ * x 5120 -> 13824: 0.5% by the estimate, 688 and 696 us with 224 rows), and
+ * over 6% if K is long (over 8192) too: the Wan FFN of 4600 rows, whose 13824
+ * -> 5120 gains 5.8% by the estimate, takes 948 us and 957 with 192 rows.
  * Measured (us, 256 rows and the pick): 300 x 5376 -> 21504 111 and 100, 778
  * 186 and 176; 1600 x 7168 -> 5376 130 and 114; 2378 x 14336 -> 5376 304 and
  * 286.
@@ -879,6 +881,7 @@ static uint32_t hk_gemm_row_blocks(uint32_t m, uint32_t columns,
                 continue;
             margin = !cut                    ? 0.02f
                      : tiles_m <= HK_GROUP_M ? 0.0f
+                     : k_steps > 128         ? 0.06f
                                              : 0.05f;
         }
         const float us = hk_gemm_estimate(jb, tiles, k_steps, cus, may_split);

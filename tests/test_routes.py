@@ -290,6 +290,9 @@ MODEL_SIZES = [
     ((9720, 5120, 13824, GELU_UP), 256, gemm_rows.TAIL),
     ((9720, 13824, 5120, STORE), 256, gemm_rows.WHOLE),
     ((9720, 5120, 15360, STORE), 256, gemm_rows.WHOLE),
+    # a long K, several bands: 948 and 957 us of the FFN with 192 rows
+    ((4600, 13824, 5120, STORE), 256, gemm_rows.TAIL),
+    ((7232, 13824, 5120, STORE), 192, gemm_rows.WHOLE),
     # more rounds: 339 and 380 us with 160 rows
     ((1400, 5376, 14336, SWIGLU_UP), 256, gemm_rows.WHOLE),
     # a last band of one row tile: 238 and 254 us with 224 rows
